@@ -696,7 +696,7 @@ static int run_shape(const mt_ctx* ctx, const mt_run_opts* o, size_t table_bytes
   s.block = ctx->tune.block ? ctx->tune.block : 256;
   s.cap = ctx->tune.stack_cap ? ctx->tune.stack_cap : 128;
   const int nwb = s.block / 64;
-  const size_t base = table_bytes + size_t(nwb) * cascade_stack_bytes(s.cap);
+  const size_t base = table_bytes + size_t(nwb) * cascade_stack_bytes(s.cap) + kNumEnergy * sizeof(double);
   const size_t lds_max = size_t(ctx->lds_max);
   if (base > lds_max) return fail(MT_E_LIMIT, "tables and stacks exceed the LDS of a workgroup");
   const int arith = o->arith, pot = ctx->tgt.potential, geo = ctx->tgt.geo.kind;

@@ -141,7 +141,7 @@ struct Params {
   unsigned long long* counters;   // kNumCounters
   double* wave_energy;            // per wave: 2 * kNumEnergy (sum, compensation)
   double* energy;                 // kNumEnergy, rare events (atomic)
-  unsigned long long *range_hist, *lat_y_hist, *lat_z_hist, *vac_hist, *repl_hist;
+  unsigned long long *range_hist, *lat_y_hist, *lat_z_hist, *vac_hist, *repl_hist;  // repl_hist = vac_hist + vac_nb + 2
   double range_x0, range_bw;
   int range_nb;
   double lat_y0, lat_z0, lat_bw;
