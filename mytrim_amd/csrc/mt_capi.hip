@@ -640,6 +640,8 @@ static_assert(sizeof(LogRecord) == sizeof(mt_record) && sizeof(mt_record) == 80,
 // ------------------------------------------------------------ run pieces
 // (shared by mt_run_cascades, mt_run_cascades_log and mt_run_cascades_noalloc)
 
+constexpr uint64_t kMaxQueue = uint64_t(1) << 27;  // most queue slots a run takes by itself
+
 // bytes per slot of each queue array (px py pz dx dy dz E key mt: 8, hist: 4, ready: 8)
 constexpr size_t kQueueFieldBytes[kQueueArrays] = {8, 8, 8, 8, 8, 8, 8, 8, 8, 4, 8};
 
@@ -658,12 +660,18 @@ static int validate_run(const mt_ctx* ctx, const mt_primaries* pk, const mt_run_
   return MT_OK;
 }
 
+// what a run needs of its primaries besides their arrays
+struct PrimaryStats {
+  double E0 = 0.0;  // total energy
+  int n = 0;        // species, each with its largest energy
+  int Z[kMaxSpecies];
+  double m[kMaxSpecies], e_max[kMaxSpecies];
+};
+
 // finite positive energies and positions, non-zero directions; the batch's
-// total and largest primary energy
-static int check_primaries(const mt_primaries* pk, double& E0, double& e_max) {
+// total energy and its species (past kMaxSpecies the run is refused later)
+static int check_primaries(const mt_primaries* pk, PrimaryStats& st) {
   const long long n_entries = pk->pka_uniform ? 1 : pk->n_hist;
-  E0 = 0.0;
-  e_max = 0.0;
   for (long long i = 0; i < n_entries; ++i) {
     if (!(pk->E[i] > 0.0) || !std::isfinite(pk->E[i])) return fail(MT_E_ARG, "primary energy must be positive and finite");
     const double* q = pk->pos + 3 * i;
@@ -672,10 +680,18 @@ static int check_primaries(const mt_primaries* pk, double& E0, double& e_max) {
       return fail(MT_E_ARG, "primary position must be finite");
     const double dd = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
     if (!(dd > 0.0) || !std::isfinite(dd)) return fail(MT_E_ARG, "primary direction must be finite and non-zero");
-    E0 += pk->E[i];
-    e_max = std::max(e_max, pk->E[i]);
+    st.E0 += pk->E[i];
+    int s = 0;
+    while (s < st.n && !(st.Z[s] == pk->Z[i] && st.m[s] == pk->m[i])) ++s;
+    if (s == st.n && st.n < kMaxSpecies) {
+      st.Z[s] = pk->Z[i];
+      st.m[s] = pk->m[i];
+      st.e_max[s] = 0.0;
+      ++st.n;
+    }
+    if (s < st.n) st.e_max[s] = std::max(st.e_max[s], pk->E[i]);
   }
-  if (pk->pka_uniform) E0 = pk->E[0] * double(pk->n_hist);
+  if (pk->pka_uniform) st.E0 = pk->E[0] * double(pk->n_hist);
   return MT_OK;
 }
 
@@ -737,13 +753,19 @@ static int run_shape(const mt_ctx* ctx, const mt_run_opts* o, size_t table_bytes
   return MT_OK;
 }
 
-// flights per cascade before any has completed: the Kinchin-Pease count
-// E / (2 Ed) of the most energetic primary against the lowest threshold
-static double flights_per_cascade0(const mt_ctx* ctx, double e_max) {
-  double ed_min = 1e300;
+// flights per cascade before any has completed: the largest estimate over the
+// primaries' species and the materials, against the lowest threshold; one
+// where no recoil is followed
+static double flights_per_cascade0(const mt_ctx* ctx, const PrimaryStats& st, const mt_run_opts* o) {
+  if (o->follow_max_gen == 0 || o->follow_max_gen == 1) return 1.0;
+  double ed_min = 1e300, f = 1.0;
   for (const HostMaterial& m : ctx->tgt.mat)
     for (const HostElement& e : m.el) ed_min = std::min(ed_min, e.Edisp);
-  return 1.0 + e_max / (2.0 * std::max(ed_min, 1.0));
+  for (const HostMaterial& m : ctx->tgt.mat)
+    for (int s = 0; s < st.n; ++s)
+      if (st.Z[s] > 0 && st.m[s] > 0.0)
+        f = std::max(f, flights_estimate(st.Z[s], st.m[s], st.e_max[s], m.az, m.am, ed_min));
+  return f;
 }
 
 // device memory of one run
@@ -806,10 +828,19 @@ static void fill_params(Params& P, const mt_ctx* ctx, const mt_primaries* pk, co
   Q.nq = nq;
   Q.sub_log2 = log2cap - lq;
   Q.sub_mask = (uint64_t(1) << Q.sub_log2) - 1;
-  P.admit_limit = (long long)(M.qcap / 4);
-  P.budget = double(M.qcap) / 2.0;
+  // a queue smaller than the batch's expected flights needs the budget kept;
+  // one wave per SIMD of a small batch admits all of it
+  const int first = std::min(sh.waves, 4 * ctx->cus);
+  P.half_share = 0.5 / sh.waves;
+  const bool roomy = double(pk->n_hist) * f_init <= 2.0 * double(M.qcap);
+  P.admit_strict = !roomy && M.qcap < kMaxQueue;
+  if (ctx->tune.primary_waves64 == 0 && !P.admit_strict && pk->n_hist <= 64ll * first) {
+    P.admit_share = int((pk->n_hist + first - 1) / first);
+    P.late_block = sh.waves > first ? first * 64 / sh.block : 0;
+  }
+  P.budget = P.admit_strict ? 12.0 * double(M.qcap) + 1024.0 * sh.waves : 0.5 * double(M.qcap);
   P.f_init = f_init;
-  P.c_floor = sh.waves;
+  P.c_floor = P.admit_strict ? std::min(512, sh.waves) : sh.waves;
   P.h_out = M.h_out;
   P.max_ic = 10000000;
   P.max_wait_ticks = (unsigned long long)(60.0 * ctx->clock_khz * 1000.0);
@@ -896,8 +927,8 @@ static int run_cascades(mt_ctx* ctx, const mt_primaries* pk, const mt_run_opts* 
   HIPCHECK(hipSetDevice(ctx->device));
   const long long n_hist = pk->n_hist;
   const long long n_entries = pk->pka_uniform ? 1 : n_hist;
-  double E0 = 0.0, e_max = 0.0;
-  if (int rc = check_primaries(pk, E0, e_max)) return rc;
+  PrimaryStats ps;
+  if (int rc = check_primaries(pk, ps)) return rc;
   std::vector<Species> species;
   std::vector<int> pka_species;
   std::string msg = collect_species(ctx->tgt, pk->Z, pk->m, n_entries, species, pka_species);
@@ -926,13 +957,13 @@ static int run_cascades(mt_ctx* ctx, const mt_primaries* pk, const mt_run_opts* 
   const int pot = ctx->tgt.potential;
   const bool log_on = lg && lg->mask != 0;
   const bool perhist = perhist_of(o, lg);
-  const double f_init = flights_per_cascade0(ctx, e_max);
+  const double f_init = flights_per_cascade0(ctx, ps, o);
 
   // queue: room for every flight of the batch up to 2^27 entries (80 B each)
   const double want = std::max(double(n_hist), 1.0) * f_init;
   uint64_t qcap = ctx->tune.queue_cap
                       ? uint64_t(ctx->tune.queue_cap)
-                      : next_pow2(uint64_t(std::min(std::max(want, 65536.0), double(uint64_t(1) << 27))));
+                      : next_pow2(uint64_t(std::min(std::max(want, 65536.0), double(kMaxQueue))));
   if (ctx->qcap != qcap) {
     for (int i = 0; i < kQueueArrays; ++i) HIPCHECK(ctx->q[i].ensure(qcap * kQueueFieldBytes[i]));
     ctx->qcap = qcap;
@@ -1091,7 +1122,7 @@ static int run_cascades(mt_ctx* ctx, const mt_primaries* pk, const mt_run_opts* 
 
   const unsigned long long* sr = static_cast<const unsigned long long*>(ctx->stage_res.p);
   const unsigned long long* ctrl = sr + kResCtrl;
-  read_results(sr, E0, ctx->clock_khz, out);
+  read_results(sr, ps.E0, ctx->clock_khz, out);
   ctx->last_t0 = ctrl[kT0];
   ctx->last_tadm = ctrl[kTAdmit];
   ctx->last_fadm = ctrl[kFlightsAtAdmit];
@@ -1692,8 +1723,8 @@ int mt_run_cascades_noalloc(mt_ctx* ctx, const mt_primaries* pk, const mt_run_op
     return fail(MT_E_LIMIT, "histograms exceed the static scratch (about 130 000 bins)");
   if (!ctx->na_scratch) return fail(MT_E_STATE, "no static scratch on this device");
   HIPCHECK(hipSetDevice(ctx->device));
-  double E0 = 0.0, e_max = 0.0;
-  if (int rc = check_primaries(pk, E0, e_max)) return rc;
+  PrimaryStats ps;
+  if (int rc = check_primaries(pk, ps)) return rc;
   Species sp[kMaxSpecies];
   int ns = 0;
   std::string msg = collect_species_into(ctx->tgt, pk->Z, pk->m, n_entries, sp, &ns);
@@ -1704,7 +1735,7 @@ int mt_run_cascades_noalloc(mt_ctx* ctx, const mt_primaries* pk, const mt_run_op
   RunShape sh;
   if (int rc = run_shape(ctx, o, tb, false, sh)) return rc;
   if (sh.waves > kNaMaxWaves) return fail(MT_E_LIMIT, "more than 16384 waves for the static scratch");
-  const double f_init = flights_per_cascade0(ctx, e_max);
+  const double f_init = flights_per_cascade0(ctx, ps, o);
 
   unsigned char* base = static_cast<unsigned char*>(ctx->na_scratch);
   int* d_sp = reinterpret_cast<int*>(base + kNaOffPka);
@@ -1776,7 +1807,7 @@ int mt_run_cascades_noalloc(mt_ctx* ctx, const mt_primaries* pk, const mt_run_op
   HIPCHECK(hipStreamSynchronize(st));
   float ms = 0.0f;
   HIPCHECK(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-  read_results(resh, E0, ctx->clock_khz, out);
+  read_results(resh, ps.E0, ctx->clock_khz, out);
   out->kernel_ms = ms;
   out->grid = sh.grid;
   out->block = sh.block;

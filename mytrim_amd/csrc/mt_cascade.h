@@ -38,7 +38,7 @@ enum Ctrl {
   kError = 64,          // error bits
   kQueueOps = 65,       // wave-level queue transfers
   // steady-state throughput of a launch, read by the launch-shape tuner:
-  // wall-clock stamp of the first wave's start, of the admission of the last
+  // wall-clock stamp of wave 0's start, of the admission of the last
   // primary, and the flights ended by then (kFlightsEnded at that moment; each
   // wave adds its ended flights in batches of up to 256)
   kT0 = 66,
@@ -126,11 +126,20 @@ struct Params {
   // work distribution
   unsigned long long* ctrl;
   Queue q;
-  long long admit_limit;        // no new primaries while the queue holds more
+  double half_share;            // 1 / (2 waves)
+  // a small batch (at most 64 primaries per SIMD): primaries a wave admits at
+  // once, without the budget (0: not small), and the first block to start late
+  // (0: none)
+  int admit_share, late_block;
+  int admit_strict;             // small queue: the budget is reserved before it is used
   // cascade budget: admitted-but-incomplete cascades times the flights per
   // cascade (f_init until 64 cascades completed, then flights ended per
-  // completed cascade, an overestimate) stays below `budget` queue entries;
-  // at least c_floor cascades may always be live
+  // completed cascade, an overestimate) stays below `budget`; at least c_floor
+  // cascades may always be live.  A queue sized for the batch is budgeted half
+  // its entries, unreserved.  In one that was given (a fixed scratch, a
+  // tuning) and is smaller, some 3 % of a live cascade's flights wait, after
+  // the lanes and stacks hold theirs: 12 times its entries and 16 a lane, each
+  // cascade reserved before it starts (admit_strict).
   double budget, f_init;
   long long c_floor;
   int* h_out;                   // per history: flights queued or running

@@ -21,6 +21,8 @@
 //     (epoch | live | idle) word; every wave leaves once all live waves are
 //     idle, every shard is empty and the primaries are used up, observed
 //     twice with the same epoch.  Waits are bounded by a wall-clock limit.
+//     Only waves that have started count as live: a grid of small blocks may
+//     not fit at once, and its last blocks then start when others have left.
 //
 // Tallies: per-lane 32-bit event counters summed over the wave at exit,
 // per-lane compensated FP64 energy sums, histogram bins in LDS (or HBM
@@ -60,6 +62,15 @@ __device__ __forceinline__ uint64_t uni64(uint64_t v) {  // lane 0's value, in s
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32));
   return ((uint64_t)hi << 32) | lo;
 }
+
+// lane src's value (src wave-uniform), in scalar registers
+__device__ __forceinline__ uint64_t lane64(uint64_t v, int src) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, src);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), src);
+  return ((uint64_t)hi << 32) | lo;
+}
+constexpr int kPollPka = 63;      // the lane that reads kPkaNext in a poll
+constexpr int kMaxPollWait = 16;  // most iterations between two polls of a wave with work
 
 // relaxed agent-scope load, made wave-uniform
 __device__ __forceinline__ uint64_t ld_relaxed(unsigned long long* p) {
@@ -269,6 +280,11 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   uint32_t* lvac = (uint32_t*)(lsum + kNumEnergy);
   uint32_t* lrepl = lvac + P.lds_hist;
   for (int i = threadIdx.x; i < 2 * P.lds_hist; i += blockDim.x) lvac[i] = 0u;
+  unsigned err = 0;
+  // live += the block's waves, performed before any of them can register idle
+  // (the barrier waits for the returned word); one addition per block, as they
+  // queue on the word's cache line
+  if (threadIdx.x == 0 && atomicAdd(&P.ctrl[kState], (unsigned long long)nwb << 16) == ~0ull) err |= kErrBadEntry;
   __syncthreads();
 
   const TableHeader* H = (const TableHeader*)lds;
@@ -285,11 +301,9 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   unsigned long long* ctrl = P.ctrl;
   const unsigned long long clk0 = (unsigned long long)clock64();
   const unsigned long long wall0 = (unsigned long long)wall_clock64();
-  if (lane == 0) {
-    atomicAdd(&ctrl[kState], 1ull << 16);  // live += 1
-    // the first wave to start stamps the launch (the words start at zero)
-    atomicCAS(&ctrl[kT0], 0ull, wall0);
-  }
+  // wave 0 stamps the launch (all waves start within a microsecond)
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(&ctrl[kT0], wall0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   // wave-uniform state
   int scount = 0;          // entries in this wave's LDS stack
@@ -300,7 +314,9 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   const int per_xcd = P.q.nq >= 8 ? P.q.nq / 8 : 1;
   const int home = (P.q.nq >= 8 ? (int)(blockIdx.x & 7u) * per_xcd + wid % per_xcd
                                 : (int)(blockIdx.x * nwb + wid)) & (P.q.nq - 1);
-  int victim = home;       // last shard this wave stole from
+  int victim = home;       // the shard after this one is polled next
+  bool pka_gone = false;   // every primary has started
+  bool first_adm = true;   // this wave has not admitted primaries yet
   // wave roles (P.primary_waves64 > 0): feeder waves admit the primaries in
   // bulk and send every recoil to the HBM queue; the others run what the
   // queue holds and admit primaries only for their idle lanes when it is
@@ -310,6 +326,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   const bool feeder_wave = roles && ((int)((blockIdx.x * nwb + wid) & 63u) < P.primary_waves64);
   bool feeding = feeder_wave;  // wave-uniform: admitted primaries at its last refill
   int poll_skip = 0;       // iterations before the shared queue is polled again
+  int poll_wait = 4;       // iterations to skip after the next poll that finds nothing
   long long peak_seen = 0; // largest queue fill this wave has reported
   unsigned long long fe_pending = 0;  // ended flights not yet added to kFlightsEnded
   // per lane: outstanding-flight count of the history before this lane's last
@@ -336,11 +353,23 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   unsigned l_newton32 = 0, l_kpvac32 = 0, l_coll32 = 0, l_ruth32 = 0, l_surr32 = 0, l_vac32 = 0;
   unsigned l_flight32 = 0, l_fate32[4] = {0u, 0u, 0u, 0u}, l_vacuum32 = 0, l_rangen32 = 0, l_coll0_32 = 0;
   double eel_s = 0.0, eel_e = 0.0, enuc_s = 0.0, enuc_e = 0.0;
-  unsigned err = 0;
 
   bool active = false;
   Flight F;
   F.ic = 0;
+
+  // Staggered start.  In a small batch the second and third wave of a SIMD
+  // start 40 us late: the first ones hold every primary by then (10 us), and
+  // two half-empty waves on a SIMD take longer than one (2000 He histories:
+  // 4.4 -> 3.4 ms).  In a larger one the blocks start over 0.27 ms: started
+  // together, the waves empty their lanes and crowd the shared words together
+  // (2e5 He histories 30 -> 25 ms, 1e6 with wave roles 100 -> 88 ms).  One
+  // nap is 1.07 us.
+  {
+    const int naps = P.admit_share == 0 ? (int)((blockIdx.x << 8) / gridDim.x)
+                     : P.late_block > 0 && (int)blockIdx.x >= P.late_block ? 38 : 0;
+    for (int z = 0; z < naps; ++z) __builtin_amdgcn_s_sleep(40);
+  }
 
   while (true) {
     // ------------------------------------------------------------ refill
@@ -358,44 +387,80 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
         const ArgPtr A = cold_args();
         // one lane loads one entry, so a batch holds at most 64
         const int want = min(64, min(cap - scount, max(n_idle, cap / 2) - scount));
-        // cascade budget (see Params): cascades that may be admitted now
-        auto budget_room = [&]() -> long long {
+        // One load by the whole wave brings the words of this poll: the
+        // primaries started, and head and tail of the home shard and of the
+        // next one to steal from (three of them when the wave has no work at
+        // all).  Read one after another a poll took up to ten trips of some
+        // 0.3 us.  More words per poll lose: a line that is read while others
+        // write it is passed between XCDs, and with all 16 shards in every
+        // poll 20 000 Cu histories took 97 ms instead of 68.
+        const int n_vict = A->q.nq == 1 ? 0 : n_idle == 64 ? min(3, A->q.nq - 1) : 1;
+        auto shard_of = [&](int v) { return v == 0 ? home : (victim + v) & (A->q.nq - 1); };
+        uint64_t snap = 0;
+        if (lane < 2 * (n_vict + 1)) {
+          const int q = shard_of(lane >> 1);
+          snap = ld_agent((const uint64_t*)&ctrl[(lane & 1) ? kQTail(q) : kQHead(q)]);
+        } else if (lane == kPollPka && !pka_gone) {
+          snap = ld_agent((const uint64_t*)&ctrl[kPkaNext]);
+        }
+        // primaries are never handed back: once all have started, the word
+        // need not be read again
+        const long long pka_left = pka_gone ? 0ll : A->n_hist - (long long)lane64(snap, kPollPka);
+        pka_gone = pka_left <= 0;
+        // Primaries this wave may admit now.  In a small batch an even share
+        // of it: the longest chains start at once, on every SIMD (64 a wave
+        // left most waves to the queue: 2000 He histories 8.5 -> 4.4 ms).
+        // Else what the cascade budget leaves (see Params), except a wave's
+        // first, which all waves make before a cascade has ended.
+        auto may_admit = [&](int most) -> long long {
+          if (A->admit_share > 0) return min(most, A->admit_share);
           const uint64_t live = ld_relaxed(&ctrl[kLive]);
           const uint64_t done = ld_relaxed(&ctrl[kCascDone]);
           const double fhat =
               done >= 64ull ? (double)ld_relaxed(&ctrl[kFlightsEnded]) / (double)done : A->f_init;
           const long long cmax = max((long long)(A->budget / fmax(fhat, 1.0)), A->c_floor);
-          return cmax - (long long)live;
+          const long long n = min((long long)most, cmax - (long long)live);
+          if (!A->admit_strict) {
+            if (!first_adm) return n;
+            first_adm = false;
+            return most;
+          }
+          if (n <= 0) return n;
+          // reserve the cascades before admitting them, so that waves that
+          // read the same count do not all take the same room
+          uint64_t was = 0;
+          if (lane == 0) was = atomicAdd(&ctrl[kLive], (unsigned long long)n);
+          const long long ok = min(n, max(0ll, cmax - (long long)bcast64(was, 0)));
+          if (lane == 0 && ok < n) atomicAdd(&ctrl[kLive], (unsigned long long)(ok - n));
+          return ok;
         };
-        const bool pka_left = ld_relaxed(&ctrl[kPkaNext]) < (unsigned long long)A->n_hist;
         long long n_adm = 0;
         // a feeder wave admits primaries while they last and the budget lets
         // it, leaving the shared queue to the others; otherwise it works like
         // any other wave
         if (feeder_wave) {
-          if (pka_left) n_adm = min((long long)want, budget_room());
+          if (pka_left > 0) n_adm = may_admit(want);
           feeding = n_adm > 0;
         }
-        // the home shard first, then up to three others (rotating victim)
         int qs = home;
         uint64_t h0 = 0, t0 = 0;
         if (!feeding) {
-          h0 = ld_relaxed(&ctrl[kQHead(qs)]);
-          t0 = ld_relaxed(&ctrl[kQTail(qs)]);
-          for (int v = 0; v < 3 && t0 <= h0 && A->q.nq > 1; ++v) {
-            victim = (victim + 1) & (A->q.nq - 1);
-            if (victim == home) victim = (victim + 1) & (A->q.nq - 1);
-            qs = victim;
-            h0 = ld_relaxed(&ctrl[kQHead(qs)]);
-            t0 = ld_relaxed(&ctrl[kQTail(qs)]);
+          for (int v = 0; v <= n_vict && t0 <= h0; ++v) {
+            qs = shard_of(v);
+            h0 = lane64(snap, 2 * v);
+            t0 = lane64(snap, 2 * v + 1);
           }
+          victim += n_vict;
         }
         const bool may_pop = t0 > h0;
         // a wave that is not feeding admits primaries when the queue has
-        // nothing for it; with roles, only as many as it has idle lanes
-        if (!feeding && !may_pop && pka_left) {
-          const int w = roles ? min(want, n_idle - scount) : want;
-          n_adm = min((long long)w, budget_room());
+        // nothing for it: as many as it has idle lanes, and without roles up
+        // to `want` while that is less than half an even share of those left
+        // (the last ones are spread over the waves)
+        if (!feeding && !may_pop && pka_left > 0) {
+          const int need = n_idle - scount;
+          const long long even = roles ? 0ll : (long long)((double)pka_left * A->half_share);
+          n_adm = may_admit(min(want, max(need, (int)min(even, 64ll))));
         }
         const bool may_pka = n_adm > 0;
         if (wave_idle && (may_pop || may_pka)) {
@@ -487,8 +552,10 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           if (lane == 0) first = atomicAdd(&ctrl[kPkaNext], (unsigned long long)n_adm);
           first = bcast64(first, 0);
           const long long got = min(n_adm, max(0ll, A->n_hist - (long long)first));
+          // a strict admission has counted its n_adm already
+          const long long uncounted = (A->admit_strict && A->admit_share == 0) ? got - n_adm : got;
+          if (lane == 0 && uncounted != 0) atomicAdd(&ctrl[kLive], (unsigned long long)uncounted);
           if (lane == 0 && got > 0) {
-            atomicAdd(&ctrl[kLive], (unsigned long long)got);
             const long long mid = A->n_hist / 2;
             if ((long long)first <= mid && (long long)first + got > mid) {  // the middle primary
               __hip_atomic_store(&ctrl[kFlightsAtHalf], (unsigned long long)ld_relaxed(&ctrl[kFlightsEnded]),
@@ -522,7 +589,12 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           }
           scount += (int)max(got, 0ll);
         }
-        if (!may_pop && !may_pka) poll_skip = 4;
+        if (may_pop || may_pka) {
+          poll_wait = 4;
+        } else {
+          poll_skip = poll_wait;
+          poll_wait = min(2 * poll_wait, kMaxPollWait);
+        }
         __builtin_amdgcn_wave_barrier();
       }
       const int take = min(n_idle, scount);

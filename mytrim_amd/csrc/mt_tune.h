@@ -1,5 +1,6 @@
-// Launch phases of a cascade launch and the rate they project for a launch of
-// more histories (host code of the autotuner, mt_autotune).
+// The flights a cascade is expected to have, and the launch phases of a cascade
+// launch with the rate they project for a launch of more histories (host code
+// of the runs and of the autotuner, mt_autotune).
 //
 // A launch ramps up until the admission of its middle primary, runs at a
 // steady rate until the admission of its last one, then drains: the last
@@ -10,11 +11,29 @@
 // steady rate.
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "mytrim_gpu.h"
 
 namespace mt {
+
+// Flights of one cascade expected from an ion (Z1, m1) of energy E in atoms
+// (Z2, m2) with displacement energy Ed, before any has been counted: the
+// damage energy T of the Lindhard partition with Robinson's fit
+// (T = E / (1 + k g(eps))) over Ed, twice the Kinchin-Pease count T / (2 Ed).
+// Full cascades ran 0.64 to 1.0 of it (H/He to Xe, 10 keV to 2 MeV); E / (2 Ed)
+// alone is 13 times too many for 100 keV He in Fe and 23 for 2 MeV C in W,
+// which left their batches with too small a share of the queue.
+inline double flights_estimate(double Z1, double m1, double E, double Z2, double m2, double Ed) {
+  const double z = std::pow(Z1, 2.0 / 3.0) + std::pow(Z2, 2.0 / 3.0);
+  const double a = 0.8853 * 0.5292 / std::sqrt(z);
+  const double eps = a * m2 * E / (Z1 * Z2 * 14.4 * (m1 + m2));
+  const double k = 0.0793 * std::pow(Z1, 2.0 / 3.0) * std::sqrt(Z2) * std::pow(m1 + m2, 1.5) /
+                   (std::pow(z, 0.75) * std::pow(m1, 1.5) * std::sqrt(m2));
+  const double g = eps + 0.40244 * std::pow(eps, 0.75) + 3.4008 * std::pow(eps, 1.0 / 6.0);
+  return 1.0 + E / (1.0 + k * g) / std::max(Ed, 1.0);
+}
 
 struct LaunchPhases {
   double kernel_s = 0.0;             // kernel time
