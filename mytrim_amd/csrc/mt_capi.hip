@@ -39,12 +39,13 @@ hipError_t scatter_launch(int arith, int potential, const MlpDev& mlp, const dou
 hipError_t ablate_launch(int mode, const MlpDev& S, const double* eps, const double* b, long long n, double* s2,
                          hipStream_t stream);
 hipError_t mlp_make_data(uint32_t seed, long long n, const MlpTriple* tri, int n_tri, double E_lo, int rect,
-                         const MlpNorm& nm, float* X, float* T, hipStream_t st);
-hipError_t mlp_train(float* p, const float* X, const float* T, long long n, int B, int epochs, float lr0,
-                     float* rec, float* part, float* g, float* m, float* v, int* t, float* batch_loss,
-                     double* losses, hipStream_t st);
-hipError_t mlp_batch_grad(const float* p, const float* X, const float* T, int B, float* rec, float* part,
-                          float* g, float* loss, hipStream_t st);
+                         const MlpNorm& nm, float* X, float* T, float* m, float* v, int* t, hipStream_t st);
+int mlp_parts(int B);
+size_t mlp_rec_floats(int B);
+hipError_t mlp_train(float* p, const float* X, const float* T, long long n, int B, int epochs, float lr0, float* rec, float* part,
+                     float* m, float* v, int* t, float* batch_loss, double* losses, hipStream_t st);
+hipError_t mlp_batch_grad(const float* p, const float* X, const float* T, int B, float* rec, float* part, float* g,
+                          float* loss, hipStream_t st);
 hipError_t mlp_pack(const float* p, uint32_t* w2bf, hipStream_t st);
 hipError_t mlp_infer_launch(const MlpDev& S, const double* eps, const double* b, long long n, double* s2,
                             hipStream_t st);
@@ -239,7 +240,7 @@ struct mt_ctx {
   HBuf f_stage;  // their pinned staging
   MBuf f_out;    // what the flight kernel writes: status words, the ion, events
   // scattering surrogate
-  DBuf mlp_p, mlp_w2bf, mlp_X, mlp_T, mlp_rec, mlp_part, mlp_g, mlp_m, mlp_v, mlp_t, mlp_bl, mlp_tri;
+  DBuf mlp_p, mlp_w2bf, mlp_X, mlp_T, mlp_rec, mlp_part, mlp_m, mlp_v, mlp_t, mlp_bl, mlp_tri;
   MlpNorm mlp_norm{};
   bool mlp_ready = false;
   int mlp_bf16 = 0;
@@ -264,8 +265,7 @@ struct mt_ctx {
     f_in.release();
     f_stage.release();
     f_out.release();
-    DBuf* ml[] = {&mlp_p,     &mlp_w2bf, &mlp_X, &mlp_T, &mlp_rec, &mlp_part,
-                  &mlp_g,     &mlp_m,    &mlp_v, &mlp_t, &mlp_bl,  &mlp_tri};
+    DBuf* ml[] = {&mlp_p, &mlp_w2bf, &mlp_X, &mlp_T, &mlp_rec, &mlp_part, &mlp_m, &mlp_v, &mlp_t, &mlp_bl, &mlp_tri};
     for (DBuf* b : ml) b->release();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -1563,9 +1563,8 @@ int mt_surrogate_train(mt_ctx* ctx, const mt_surrogate_opts* o, float* params, d
   HIPCHECK(ctx->mlp_p.ensure(kMlpParams * sizeof(float)));
   HIPCHECK(ctx->mlp_X.ensure(size_t(n) * kMlpIn * sizeof(float)));
   HIPCHECK(ctx->mlp_T.ensure(size_t(n) * sizeof(float)));
-  HIPCHECK(ctx->mlp_rec.ensure(size_t(B) * kMlpRecord * sizeof(float)));
-  HIPCHECK(ctx->mlp_part.ensure(size_t((B + kMlpGradChunk - 1) / kMlpGradChunk) * (kMlpParams + 1) * sizeof(float)));
-  HIPCHECK(ctx->mlp_g.ensure((kMlpParams + 1) * sizeof(float)));
+  HIPCHECK(ctx->mlp_rec.ensure(mlp_rec_floats(B) * sizeof(float)));
+  HIPCHECK(ctx->mlp_part.ensure(size_t(mlp_parts(B)) * (kMlpParams + 1) * sizeof(float)));
   HIPCHECK(ctx->mlp_m.ensure(kMlpParams * sizeof(float)));
   HIPCHECK(ctx->mlp_v.ensure(kMlpParams * sizeof(float)));
   HIPCHECK(ctx->mlp_t.ensure(sizeof(int)));
@@ -1573,15 +1572,12 @@ int mt_surrogate_train(mt_ctx* ctx, const mt_surrogate_opts* o, float* params, d
   HIPCHECK(ctx->mlp_tri.ensure(tri.size() * sizeof(MlpTriple)));
   HIPCHECK(hipMemcpyAsync(ctx->mlp_tri.p, tri.data(), tri.size() * sizeof(MlpTriple), hipMemcpyHostToDevice, st));
   HIPCHECK(hipMemcpyAsync(ctx->mlp_p.p, params, kMlpParams * sizeof(float), hipMemcpyHostToDevice, st));
-  HIPCHECK(hipMemsetAsync(ctx->mlp_m.p, 0, kMlpParams * sizeof(float), st));
-  HIPCHECK(hipMemsetAsync(ctx->mlp_v.p, 0, kMlpParams * sizeof(float), st));
-  HIPCHECK(hipMemsetAsync(ctx->mlp_t.p, 0, sizeof(int), st));
   HIPCHECK(mlp_make_data(o->seed, n, ctx->mlp_tri.as<MlpTriple>(), int(tri.size()), o->E_min, o->sampling, nm,
-                         ctx->mlp_X.as<float>(), ctx->mlp_T.as<float>(), st));
+                         ctx->mlp_X.as<float>(), ctx->mlp_T.as<float>(), ctx->mlp_m.as<float>(),
+                         ctx->mlp_v.as<float>(), ctx->mlp_t.as<int>(), st));
   HIPCHECK(mlp_train(ctx->mlp_p.as<float>(), ctx->mlp_X.as<float>(), ctx->mlp_T.as<float>(), n, B, o->epochs,
-                     float(o->lr), ctx->mlp_rec.as<float>(), ctx->mlp_part.as<float>(), ctx->mlp_g.as<float>(),
-                     ctx->mlp_m.as<float>(),
-                     ctx->mlp_v.as<float>(), ctx->mlp_t.as<int>(), ctx->mlp_bl.as<float>(), epoch_loss, st));
+                     float(o->lr), ctx->mlp_rec.as<float>(), ctx->mlp_part.as<float>(), ctx->mlp_m.as<float>(), ctx->mlp_v.as<float>(),
+                     ctx->mlp_t.as<int>(), ctx->mlp_bl.as<float>(), epoch_loss, st));
   HIPCHECK(hipMemcpyAsync(params, ctx->mlp_p.p, kMlpParams * sizeof(float), hipMemcpyDeviceToHost, st));
   HIPCHECK(hipStreamSynchronize(st));
   return MT_OK;
@@ -1688,15 +1684,15 @@ int mt_surrogate_grad(mt_ctx* ctx, const mt_surrogate_opts* o, const float* para
   HIPCHECK(ctx->scratch_a.ensure(kMlpParams * sizeof(float)));
   HIPCHECK(ctx->scratch_b.ensure(X.size() * sizeof(float)));
   HIPCHECK(ctx->scratch_c.ensure(T.size() * sizeof(float) + 16));
-  HIPCHECK(ctx->scratch_d.ensure(size_t(n) * kMlpRecord * sizeof(float)));
   HIPCHECK(ctx->scratch_e.ensure((kMlpParams + 1) * sizeof(float)));
-  HIPCHECK(ctx->mlp_part.ensure(size_t((n + kMlpGradChunk - 1) / kMlpGradChunk) * (kMlpParams + 1) * sizeof(float)));
+  HIPCHECK(ctx->mlp_rec.ensure(mlp_rec_floats(n) * sizeof(float)));
+  HIPCHECK(ctx->mlp_part.ensure(size_t(mlp_parts(n)) * (kMlpParams + 1) * sizeof(float)));
   HIPCHECK(hipMemcpyAsync(ctx->scratch_a.p, params, kMlpParams * sizeof(float), hipMemcpyHostToDevice, st));
   HIPCHECK(hipMemcpyAsync(ctx->scratch_b.p, X.data(), X.size() * sizeof(float), hipMemcpyHostToDevice, st));
   HIPCHECK(hipMemcpyAsync(ctx->scratch_c.p, T.data(), T.size() * sizeof(float), hipMemcpyHostToDevice, st));
   float* g = ctx->scratch_e.as<float>();
   HIPCHECK(mlp_batch_grad(ctx->scratch_a.as<float>(), ctx->scratch_b.as<float>(), ctx->scratch_c.as<float>(), n,
-                          ctx->scratch_d.as<float>(), ctx->mlp_part.as<float>(), g, g + kMlpParams, st));
+                          ctx->mlp_rec.as<float>(), ctx->mlp_part.as<float>(), g, g + kMlpParams, st));
   float lf = 0.0f;
   HIPCHECK(hipMemcpyAsync(grad, g, kMlpParams * sizeof(float), hipMemcpyDeviceToHost, st));
   HIPCHECK(hipMemcpyAsync(&lf, g + kMlpParams, sizeof(float), hipMemcpyDeviceToHost, st));

@@ -21,10 +21,6 @@ constexpr int kOffB2 = kOffW2 + kMlpH * kMlpH;  // b2[k]
 constexpr int kOffW3 = kOffB2 + kMlpH;        // W3[k]
 constexpr int kOffB3 = kOffW3 + kMlpH;        // b3
 constexpr int kMlpParams = kOffB3 + 1;        // 4481
-// floats per training sample written by the forward/backward kernel
-constexpr int kMlpRecord = 4 + 4 * kMlpH + 1;
-// samples per partial sum of the gradient reduction
-constexpr int kMlpGradChunk = 128;
 
 // input / output scaling and the trained domain
 struct MlpNorm {

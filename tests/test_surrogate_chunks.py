@@ -1,0 +1,33 @@
+"""Edges of the gradient kernel's chunks of 128 samples (tiles of 16): batches that
+end inside a tile, fill a tile, fill a chunk, and give many chunks."""
+import numpy as np
+import pytest
+
+import mlp_ref as M
+from mytrim_amd import configs, gpu
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 127, 128, 129, 20011])
+def test_gradient_chunks(n):
+    prob = configs.c5_c_w(10, seed=43)
+    e = gpu.Engine(0)
+    try:
+        e.set_target(prob)
+        opts = gpu.Engine.surrogate_opts(prob)
+        norm = e.surrogate_norm(opts)
+        rng = np.random.default_rng(n)
+        p = gpu.Engine.surrogate_init(n)
+        eps = np.exp(rng.uniform(np.log(norm["eps_lo"]), np.log(norm["eps_hi"]), n))
+        b = norm["b_hi"] * np.sqrt(rng.random(n))
+        ls2 = -8.0 + 8.0 * rng.uniform(-1.0, 1.0, n)
+        g, loss = e.surrogate_grad(opts, p, eps, b, ls2)
+        ref_loss, ref = M.loss_grad(p, M.inputs(norm, eps, b), M.target(norm, ls2))
+        # single precision: inputs, tanh (hardware exp and reciprocal, 2 ulp) and
+        # products each within 2.5e-7 relative, a chain of a dozen, 4481 sums
+        assert np.linalg.norm(g - ref) <= 3e-6 * np.linalg.norm(ref) + 1e-9
+        assert loss == pytest.approx(ref_loss, rel=3e-6)
+        again, _ = e.surrogate_grad(opts, p, eps, b, ls2)
+        assert np.array_equal(g, again)
+    finally:
+        e.close()
