@@ -159,7 +159,21 @@ __device__ __forceinline__ R getrstop(const TableView& T, int s, int k, R E) {
 // S = sum c_i exp(-d_i r) and D = sum c_i d_i exp(-d_i r) = -S'(r), for the
 // universal (POT 0), Moliere (1) and C-Kr (2) screenings of trim.C:205-232.
 // The reference's v = V and v1 = V' follow as v = S / r, v1 = -(v + D) / r.
-template <typename R, int POT>
+// QUAD: every lane of the wave has the same r (one flight per wave); the lanes
+// of a quad evaluate one exponential each, the same operations, side by side.
+__device__ __forceinline__ double quad_lane(double x, int which) {  // the quad's lane 0..3
+  const long long v = __double_as_longlong(x);
+  int lo = (int)v, hi = (int)(v >> 32);
+  switch (which) {  // DPP quad_perm(which, which, which, which)
+    case 0: lo = __builtin_amdgcn_mov_dpp(lo, 0x00, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0x00, 0xf, 0xf, true); break;
+    case 1: lo = __builtin_amdgcn_mov_dpp(lo, 0x55, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0x55, 0xf, 0xf, true); break;
+    case 2: lo = __builtin_amdgcn_mov_dpp(lo, 0xaa, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0xaa, 0xf, 0xf, true); break;
+    default: lo = __builtin_amdgcn_mov_dpp(lo, 0xff, 0xf, 0xf, true); hi = __builtin_amdgcn_mov_dpp(hi, 0xff, 0xf, 0xf, true);
+  }
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <typename R, int POT, bool QUAD = false>
 __device__ __forceinline__ void screening(R r, R& S, R& D) {
   if (POT == 1) {
     const R ex1 = m_exp(K(-0.3) * r);
@@ -174,10 +188,24 @@ __device__ __forceinline__ void screening(R r, R& S, R& D) {
     S = K(0.191) * ex1 + K(0.474) * ex2 + K(0.335) * ex3;
     D = K(0.531865) * ex1 + K(0.30181) * ex2 + K(0.6437) * ex3;
   } else {
-    const R ex1 = K(0.18175) * m_exp(K(-3.1998) * r);
-    const R ex2 = K(0.50986) * m_exp(K(-0.94229) * r);
-    const R ex3 = K(0.28022) * m_exp(K(-0.4029) * r);
-    const R ex4 = K(0.028171) * m_exp(K(-0.20162) * r);
+    R e1, e2, e3, e4;
+    if constexpr (QUAD) {
+      const int l = threadIdx.x & 3;
+      const R e = m_exp((l == 0 ? K(-3.1998) : l == 1 ? K(-0.94229) : l == 2 ? K(-0.4029) : K(-0.20162)) * r);
+      e1 = quad_lane(e, 0);
+      e2 = quad_lane(e, 1);
+      e3 = quad_lane(e, 2);
+      e4 = quad_lane(e, 3);
+    } else {
+      e1 = m_exp(K(-3.1998) * r);
+      e2 = m_exp(K(-0.94229) * r);
+      e3 = m_exp(K(-0.4029) * r);
+      e4 = m_exp(K(-0.20162) * r);
+    }
+    const R ex1 = K(0.18175) * e1;
+    const R ex2 = K(0.50986) * e2;
+    const R ex3 = K(0.28022) * e3;
+    const R ex4 = K(0.028171) * e4;
     S = ex1 + ex2 + ex3 + ex4;
     D = K(3.1998) * ex1 + K(0.94229) * ex2 + K(0.4029) * ex3 + K(0.20162) * ex4;
   }
@@ -190,14 +218,14 @@ __device__ __forceinline__ void screening(R r, R& S, R& D) {
 //   f = b^2 (1/r) + S / eps - r,  f' = -b^2 (1/r)^2 - D / eps - 1.
 // Returns the iteration count; v and v1 are those of the last r evaluated
 // (before its update), as in the reference.
-template <typename R, int POT>
+template <typename R, int POT, bool QUAD = false>
 __device__ __forceinline__ int apsis(R eps, R b, R& r, R& v, R& v1) {
   const R bb = b * b, ieps = m_rcp(eps);
   R q;
   int it = 0;
   do {
     R S, D;
-    screening<R, POT>(r, S, D);
+    screening<R, POT, QUAD>(r, S, D);
     const R ir = m_rcp(r);
     v = S * ir;
     v1 = -(v + D) * ir;
@@ -246,7 +274,7 @@ __device__ __forceinline__ void magic(R eps, R lb, R& aa, R& ff) {  // lb = log 
 }
 
 // trim.C:172-272
-template <typename R, int POT>
+template <typename R, int POT, bool QUAD = false>
 __device__ __forceinline__ void scatter(R eps, R b, R leps, R& s2, R& ct, R& st, int& iters) {
   if (eps > K(10.0)) {
     s2 = m_rcp(K(1.0) + (K(1.0) + b * (K(1.0) + b)) * sq(K(2.0) * eps * b));
@@ -264,7 +292,7 @@ __device__ __forceinline__ void scatter(R eps, R b, R leps, R& s2, R& ct, R& st,
     if (rr >= b) r = rr;
   }
   R v, v1;
-  const int it = apsis<R, POT>(eps, b, r, v, v1);
+  const int it = apsis<R, POT, QUAD>(eps, b, r, v, v1);
   const R roc = K(-2.0) * (eps - v) * m_rcp(v1);
   R aa, ff;
   magic<R, POT>(eps, lb, aa, ff);
