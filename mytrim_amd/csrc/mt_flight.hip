@@ -284,7 +284,7 @@ __global__ void __launch_bounds__(256) flight_kernel(FlightParams P) {
     for (int i = 0; i < 3; ++i) lost |= cut[i] & ((ion.pos[i] > w[i]) | (ion.pos[i] < 0.0));
     const int above = rE > r.Edisp - r.Elbind, moves = ion.E > r.Edisp;
     const int fate = lost ? 2 : above;
-    const int wild = (ion.E - ion.E == 0.0) & (ion.pos[0] - ion.pos[0] == 0.0) ? 0 : 1;
+    const int vac = (lost == 0) & above & moves;
     ion.state = lost ? 4 : above ? (moves ? 0 : ion.Z == r.Z ? 1 : 2) : ion.E < ion.Ef ? 3 : 0;
     iu = r.iu;
     r2 = r.r2;
