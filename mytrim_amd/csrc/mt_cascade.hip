@@ -222,7 +222,7 @@ __device__ __forceinline__ void physics(const TableView& T, int sp, int k, doubl
     // impact parameter and target atom (trim.C:143-160)
     const double p = pmax * m_sqrt(u53(blk.x, blk.y));
     eps = ec.fi * E;
-    const double b = p * m_rcp(ec.ai);
+    const double b = p * ec.inv_ai;
     // electronic loss along ls (trim.C:166-170) and scattering (trim.C:172-272)
     dee = ls * getrstop<double>(T, sp, k, E, lE);
     scatter<double, POT>(eps, b, lE + ec.ln_fi, s2, ct, st, it);
@@ -285,6 +285,12 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   // (the barrier waits for the returned word); one addition per block, as they
   // queue on the word's cache line
   if (threadIdx.x == 0 && atomicAdd(&P.ctrl[kState], (unsigned long long)nwb << 16) == ~0ull) err |= kErrBadEntry;
+  __syncthreads();
+  {  // reciprocals the collisions share, by the arithmetic that they used for each
+    const TableHeader* h = (const TableHeader*)lds;
+    ElemConst* el = (ElemConst*)(lds + h->off_el);
+    for (int i = threadIdx.x; i < h->n_species * h->n_el; i += blockDim.x) el[i].inv_ai = m_rcp(el[i].ai);
+  }
   __syncthreads();
 
   const TableHeader* H = (const TableHeader*)lds;
@@ -787,6 +793,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           lg_follow = lg_above && (P.follow_max_gen < 0 || F.gen + 1 < P.follow_max_gen);
         }
         // fate of recoil and ion (trim.C:357-411)
+        double enuc = 0.0;  // to nuclear losses, added where the branches meet
         if (lost) {
           state = 4;
           atomicAdd(&lsum[eElost], F.E);
@@ -795,7 +802,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           const bool follow = C->follow_max_gen < 0 || F.gen + 1 < C->follow_max_gen;
           if (follow) {
             push = true;
-            kadd(enuc_s, enuc_e, ec.Elbind);
+            enuc = ec.Elbind;
             const double inv = fx_rsqrt(rdx * rdx + rdy * rdy + rdz * rdz);
             rdx *= inv;
             rdy *= inv;
@@ -831,15 +838,16 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           } else {
             // replacementCollision (trim.C:388-395)
             state = (H->species[F.sp].Z == ec.Z) ? 1 : 2;
-            kadd(enuc_s, enuc_e, F.E);
+            enuc += F.E;
           }
         } else {
-          kadd(enuc_s, enuc_e, rE + ec.Elbind);
+          enuc = rE + ec.Elbind;
           if (F.E < C->Ef) {
             state = 3;
-            kadd(enuc_s, enuc_e, F.E);
+            enuc += F.E;
           }
         }
+        kadd(enuc_s, enuc_e, enuc);
         ended = state > 0;
         if (F.ic >= P.max_ic && !ended) {
           err |= kErrRunaway;

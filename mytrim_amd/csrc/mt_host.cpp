@@ -80,6 +80,22 @@ static StopConst make_stop(const std::vector<CoefRow>& coef, int z1, double m_io
   c.yr_lo = vrmin / c.cbrt2_fz1;
   c.yr_branch = std::max(yrmin, vrmin / c.cbrt2_fz1);
   c.vk = 3.0 * vfermi / 4.0;
+  {
+    // the velocity v (in Fermi velocities) at which vr, increasing in v, comes
+    // within 1e-5 of the branch's limit: far above single precision's rounding
+    auto vr = [&](double v) {
+      return v >= 1.0 ? v * vfermi * (1.0 + 1.0 / (5.0 * v * v))
+                      : c.vk * (1.0 + v * v / 1.5 - v * v * v * v / 15.0);
+    };
+    const double limit = c.yr_branch * c.cbrt2_fz1 * (1.0 - 1e-5);
+    double lo = 0.0, hi = 1.0;
+    while (vr(hi) < limit && hi < 1e6) hi *= 2.0;
+    for (int i = 0; i < 60; ++i) {
+      const double mid = 0.5 * (lo + hi);
+      (vr(mid) < limit ? lo : hi) = mid;
+    }
+    c.e_low = vr(0.0) < limit ? 25.0 * lo * lo * vfermi * vfermi * (1.0 - 1e-6) : 0.0;
+  }
   c.bq = (std::min(0.43, std::max(0.32, 0.12 + 0.025 * fz1))) / c.cbrt_fz1;
   c.l0k = std::min(1.2, 0.6 + fz1 / 30.0);
   c.q1 = std::max(0.0, 0.9 - 0.025 * fz1);

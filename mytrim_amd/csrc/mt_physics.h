@@ -73,6 +73,11 @@ __device__ __forceinline__ R rpstop(const StopConst& c, R e, R le) {  // materia
   return sp;
 }
 
+//
+// The Z1^3 terms 1 + c exp(-(7.6 - log e)^2), c at most 0.036, are exactly 1
+// for log e under 1.8 (the addend is under 2^-53): a wave of slow ions skips
+// their exponential.
+constexpr double kZ1cNone = 1.8;
 template <typename R>
 __device__ __forceinline__ R rstop(const StopConst& c, R E, R lE) {  // material.C:161-282
   const R e = (K(0.001) * E) * R(c.inv_m1);
@@ -89,25 +94,32 @@ __device__ __forceinline__ R rstop(const StopConst& c, R E, R lE) {  // material
     R a = K(0.2865) + K(0.1266) * b - K(0.001429) * b2 + K(0.02402) * b * b2 - K(0.01135) * b4 +
           K(0.001475) * b4 * b;
     R heh = K(1.0) - m_exp(-mn(K(30.0), a));
-    a = K(1.0) + R(c.he_k) * m_exp(-sq(K(7.6) - b));
-    heh *= a * a;
+    if (!(b < K(kZ1cNone))) {
+      a = K(1.0) + R(c.he_k) * m_exp(-sq(K(7.6) - b));
+      heh *= a * a;
+    }
     se = rpstop(c, he, b) * heh * K(4.0);
     if (e <= he0) se *= m_sqrt(e);
   } else {
     const R vf = R(c.vfermi);
-    const R v = m_sqrt(e * K(0.04)) * R(c.inv_vfermi);
-    const R v2 = v * v;
-    R vr;
-    if (v >= K(1.0))
-      vr = v * vf * (K(1.0) + m_rcp(K(5.0) * v2));
-    else
-      vr = R(c.vk) * (K(1.0) + v2 * K(2.0 / 3.0) - v2 * v2 * K(1.0 / 15.0));
-    R yr = mx(K(0.13), vr * R(c.inv_cbrt2_fz1));
-    yr = mx(yr, R(c.yr_lo));
     // yr is at least yr_branch = max(yrmin, vrmin / cbrt2 fz1); the
     // low-velocity branch (yr <= yr_branch) has yr = yr_branch, where q, l
-    // and the effective-charge factor are per-(ion, element) constants
-    const bool low = yr <= R(c.yr_branch);
+    // and the effective-charge factor are per-(ion, element) constants.  Below
+    // e_low it is taken for sure, and yr need not be worked out
+    bool low = true;
+    R yr = K(0.0);
+    if (!(e < R(c.e_low))) {
+      const R v = m_sqrt(e * K(0.04)) * R(c.inv_vfermi);
+      const R v2 = v * v;
+      R vr;
+      if (v >= K(1.0))
+        vr = v * vf * (K(1.0) + m_rcp(K(5.0) * v2));
+      else
+        vr = R(c.vk) * (K(1.0) + v2 * K(2.0 / 3.0) - v2 * v2 * K(1.0 / 15.0));
+      yr = mx(K(0.13), vr * R(c.inv_cbrt2_fz1));
+      yr = mx(yr, R(c.yr_lo));
+      low = yr <= R(c.yr_branch);
+    }
     R zeta;
     if (low) {
       zeta = R(c.zeta_lo);
@@ -128,8 +140,10 @@ __device__ __forceinline__ R rstop(const StopConst& c, R E, R lE) {  // material
       const R l = mx(l1, l0 * R(c.lfctr));
       zeta = q + R(c.zk) * (K(1.0) - q) * m_log(K(1.0) + sq(l * vf * K(4.0 / 1.919)));
     }
-    const R a = -sq(K(7.6) - mx(K(0.0), le));
-    zeta *= K(1.0) + R(c.z3) * m_exp(a);
+    if (!(le < K(kZ1cNone))) {
+      const R a = -sq(K(7.6) - mx(K(0.0), le));
+      zeta *= K(1.0) + R(c.z3) * m_exp(a);
+    }
     if (low)
       se = R(c.sp_low) * sq(zeta * R(c.fz1)) * m_exp(R(c.power) * (le - R(c.ln_eee)));
     else

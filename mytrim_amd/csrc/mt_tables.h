@@ -28,6 +28,7 @@ struct ElemConst {  // per (species, element)
   double t;         // normalised stoichiometric fraction
   double fi, ai, ec, my;
   double ln_fi;     // log fi: log eps = log E + ln_fi
+  double inv_ai;    // the kernel's own reciprocal of ai, set in its copy (LDS)
   double Edisp, Elbind;
   int Z;
   int recoil_species;
@@ -41,6 +42,7 @@ struct StopConst {  // per (species, element): rstop(ion, Z2)
   double cbrt_fz1, cbrt2_fz1;
   double yr_lo;                 // vrmin / cbrt2_fz1
   double yr_branch;             // max(yrmin, vrmin / cbrt2_fz1)
+  double e_low;                 // below this e (keV/amu) yr is yr_branch (0: nowhere)
   double vk;                    // 3 vfermi / 4
   double bq;                    // min(0.43, max(0.32, 0.12 + 0.025 Z1)) / cbrt(Z1)
   double l0k;                   // min(1.2, 0.6 + Z1/30)
