@@ -322,6 +322,10 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
                                 : (int)(blockIdx.x * nwb + wid)) & (P.q.nq - 1);
   int victim = home;       // the shard after this one is polled next
   bool pka_gone = false;   // every primary has started
+  // A history's outstanding flights are counted for the cascade budget only: not
+  // in a small batch, and not once every primary has started.  Counting takes
+  // two HBM atomics per flight, and a push to the queue waits for one.
+  bool counting = P.admit_share == 0;
   bool first_adm = true;   // this wave has not admitted primaries yet
   // wave roles (P.primary_waves64 > 0): feeder waves admit the primaries in
   // bulk and send every recoil to the HBM queue; the others run what the
@@ -413,6 +417,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
         // need not be read again
         const long long pka_left = pka_gone ? 0ll : A->n_hist - (long long)lane64(snap, kPollPka);
         pka_gone = pka_left <= 0;
+        if (pka_gone) counting = false;
         // Primaries this wave may admit now.  In a small batch an even share
         // of it: the longest chains start at once, on every SIMD (64 a wave
         // left most waves to the queue: 2000 He histories 8.5 -> 4.4 ms).
@@ -656,7 +661,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           break;
         }
         if (ld_relaxed(&ctrl[kError]) != 0ull) break;  // a wave aborted the run
-        close_pending();
+        if (counting) close_pending();
         // back off (up to ~30 us) so idle waves do not crowd the control words
         for (int z = 0; z < backoff; ++z) __builtin_amdgcn_s_sleep(127);
         backoff = min(2 * backoff, 8);
@@ -960,7 +965,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
       const uint32_t meta = (uint32_t)rsp | ((uint32_t)(F.gen + 1) << 8);
       const uint64_t rkey = child_key(F.key, (uint32_t)F.ic);
       int inc_old = 1;
-      if (push) {
+      if (counting && push) {
         const ArgPtr C1 = cold_args();
         int* ho = &C1->h_out[F.hist - (uint32_t)C1->hist0];
         if (over)  // returning: performed before the entry is published (below)
@@ -1078,11 +1083,13 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
         atomicOr((unsigned int*)&ctrl[kError], (unsigned)kErrNonFinite);
       // the decrement's old value is read one iteration later (close_pending)
       // so its latency overlaps the next collision
-      close_pending();
-      if (fin) {
-        const ArgPtr C2 = cold_args();
-        pend_old = atomicAdd(&C2->h_out[F.hist - (uint32_t)C2->hist0], -1);
-        pend = true;
+      if (counting) {
+        close_pending();
+        if (fin) {
+          const ArgPtr C2 = cold_args();
+          pend_old = atomicAdd(&C2->h_out[F.hist - (uint32_t)C2->hist0], -1);
+          pend = true;
+        }
       }
       fe_pending += __popcll(fin_m);
       if (lane == 0 && fe_pending >= 256ull) atomicAdd(&ctrl[kFlightsEnded], fe_pending);
