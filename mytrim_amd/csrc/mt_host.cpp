@@ -90,7 +90,7 @@ static StopConst make_stop(const std::vector<CoefRow>& coef, int z1, double m_io
     const double limit = c.yr_branch * c.cbrt2_fz1 * (1.0 - 1e-5);
     double lo = 0.0, hi = 1.0;
     while (vr(hi) < limit && hi < 1e6) hi *= 2.0;
-    for (int i = 0; i < 60; ++i) {
+    for (int i = 0; i < 24; ++i) {
       const double mid = 0.5 * (lo + hi);
       (vr(mid) < limit ? lo : hi) = mid;
     }
