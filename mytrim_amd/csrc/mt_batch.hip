@@ -4,7 +4,9 @@
 // ARITH selects the device functions of a cascade precision mode: 0 the FP64
 // twins of the reference, 1 the single-precision ones, 2 the single-precision
 // ones with the learned scattering map in front (the stopping of modes 1 and
-// 2 is the same).  Inputs and outputs are doubles in every mode.
+// 2 is the same).  Inputs and outputs are doubles in every mode, in host memory
+// that the kernels read and write directly: a batch takes one launch and no
+// copy, and the link (56 GB/s) bounds a large one, 44 B a pair.
 #include <hip/hip_runtime.h>
 
 #include "mt_mlp.h"
@@ -14,9 +16,17 @@
 
 namespace mt {
 
+// lds_bytes > 0: the tables lie in host memory too and each block brings them to
+// LDS in one burst (read where they are used, each constant would cross the link)
 template <int ARITH>
-__global__ void __launch_bounds__(256) stopping_kernel(const unsigned char* blob, int s, int k, const double* E,
-                                                       long long n, double* out) {
+__global__ void __launch_bounds__(256) stopping_kernel(const unsigned char* blob, int lds_bytes, int s, int k,
+                                                       const double* E, long long n, double* out) {
+  extern __shared__ __align__(16) unsigned char lds_tables[];
+  if (lds_bytes > 0) {
+    for (int i = threadIdx.x; i < lds_bytes / 16; i += blockDim.x) ((uint4*)lds_tables)[i] = ((const uint4*)blob)[i];
+    __syncthreads();
+    blob = lds_tables;
+  }
   const TableHeader* H = (const TableHeader*)blob;
   TableView T;
   T.n_species = H->n_species;
@@ -64,12 +74,14 @@ static int grid_for(long long n) {
   return (int)(g < 65536 ? (g > 0 ? g : 1) : 65536);
 }
 
-hipError_t stopping_launch(int arith, const unsigned char* tables, int species, int mat, const double* E, long long n,
-                           double* out, hipStream_t stream) {
+hipError_t stopping_launch(int arith, const unsigned char* tables, int lds_bytes, int species, int mat, const double* E,
+                           long long n, double* out, hipStream_t stream) {
   if (arith == 0)
-    hipLaunchKernelGGL(stopping_kernel<0>, dim3(grid_for(n)), dim3(256), 0, stream, tables, species, mat, E, n, out);
+    hipLaunchKernelGGL(stopping_kernel<0>, dim3(grid_for(n)), dim3(256), lds_bytes, stream, tables, lds_bytes, species,
+                       mat, E, n, out);
   else
-    hipLaunchKernelGGL(stopping_kernel<1>, dim3(grid_for(n)), dim3(256), 0, stream, tables, species, mat, E, n, out);
+    hipLaunchKernelGGL(stopping_kernel<1>, dim3(grid_for(n)), dim3(256), lds_bytes, stream, tables, lds_bytes, species,
+                       mat, E, n, out);
   return hipGetLastError();
 }
 

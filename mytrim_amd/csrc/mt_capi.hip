@@ -32,8 +32,8 @@ hipError_t zero_spans_launch(const ZeroSpans& z, hipStream_t st);
 hipError_t flush_energy_launch(const double* we, int waves, double* out, hipStream_t st);
 hipError_t primary_species_launch(const SpeciesList& L, const int* Z, const double* m, long long n, int* out,
                                   hipStream_t st);
-hipError_t stopping_launch(int arith, const unsigned char* tables, int species, int mat, const double* E, long long n,
-                           double* out, hipStream_t stream);
+hipError_t stopping_launch(int arith, const unsigned char* tables, int lds_bytes, int species, int mat, const double* E,
+                           long long n, double* out, hipStream_t stream);
 hipError_t scatter_launch(int arith, int potential, const MlpDev& mlp, const double* eps, const double* b, long long n,
                           double* s2, double* ct, double* st, int* iters, hipStream_t stream);
 hipError_t ablate_launch(int mode, const MlpDev& S, const double* eps, const double* b, long long n, double* s2,
@@ -239,12 +239,17 @@ struct mt_ctx {
   DBuf f_in;     // single flight: the ion and the caller's uniforms
   HBuf f_stage;  // their pinned staging
   MBuf f_out;    // what the flight kernel writes: status words, the ion, events
+  // function batches: two chunks of inputs and outputs (the first one's buffer
+  // begins with the tables) in memory that the kernels address, and an event
+  // for each
+  MBuf b_io[2];
+  hipEvent_t b_ev[2] = {nullptr, nullptr};
   // scattering surrogate
   DBuf mlp_p, mlp_w2bf, mlp_X, mlp_T, mlp_rec, mlp_part, mlp_m, mlp_v, mlp_t, mlp_bl, mlp_tri;
   MlpNorm mlp_norm{};
   bool mlp_ready = false;
   int mlp_bf16 = 0;
-  DBuf scratch_a, scratch_b, scratch_c, scratch_d, scratch_e;
+  DBuf scratch_a, scratch_b, scratch_c, scratch_e;
   DBuf log_rec, log_map, log_tr;  // event records, TrimVacMap map, layer transport
   // mt_run_cascades_noalloc: the device's static scratch and a host buffer
   // for the table blob, sized once here
@@ -254,7 +259,7 @@ struct mt_ctx {
   ~mt_ctx() {
     graph.release();
     DBuf* all[] = {&tables, &sh, &cl, &cx, &cy, &cz, &cr, &occ, &occ_rank, &occ_off, &occ_idx, &pka_sp, &pka_E, &pka_pos, &pka_dir, &res,
-                   &wave_energy, &hist_all, &h_out, &scratch_a, &scratch_b, &scratch_c, &scratch_d, &scratch_e,
+                   &wave_energy, &hist_all, &h_out, &scratch_a, &scratch_b, &scratch_c, &scratch_e,
                    &log_rec, &log_map, &log_tr};
     for (DBuf* b : all) b->release();
     stage_res.release();
@@ -265,6 +270,9 @@ struct mt_ctx {
     f_in.release();
     f_stage.release();
     f_out.release();
+    for (auto& b : b_io) b.release();
+    for (auto& e : b_ev)
+      if (e) (void)hipEventDestroy(e);
     DBuf* ml[] = {&mlp_p, &mlp_w2bf, &mlp_X, &mlp_T, &mlp_rec, &mlp_part, &mlp_m, &mlp_v, &mlp_t, &mlp_bl, &mlp_tri};
     for (DBuf* b : ml) b->release();
     if (ev0) (void)hipEventDestroy(ev0);
@@ -272,6 +280,49 @@ struct mt_ctx {
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
+
+// A batch of n elements through the mapped chunks: `fill` copies elements
+// [first, first + count) in, `launch` runs the kernel on them, `drain` copies
+// the results out; a chunk's kernel runs while the other chunk is copied.  One
+// launch and one wait for a small batch: a table of 97 stopping powers takes
+// 22 us, with three copies around its kernel it took 36 us (launch and wait
+// alone are 11 us).  No page of the caller's arrays is pinned for a large one:
+// 250 001 deflections take 0.91 ms against 0.99 ms.  Chunks of 2^16: the copies
+// of one take as long as the kernel of the other.  A context's first batch also
+// pays for the pinned buffer (11 us for any size up to 256 KiB).
+constexpr long long kBatchChunk = 1ll << 16;
+template <class Fill, class Launch, class Drain>
+static int run_batch(mt_ctx* ctx, long long n, size_t bytes_each, const std::vector<unsigned char>& tables, Fill fill,
+                     Launch launch, Drain drain) {
+  hipStream_t st = ctx->stream;
+  const long long chunks = (n + kBatchChunk - 1) / kBatchChunk;
+  const size_t bytes = size_t(std::min(n, kBatchChunk)) * bytes_each;
+  const size_t off[2] = {(tables.size() + 255) & ~size_t(255), 0};  // where each buffer's chunk begins
+  for (int h = 0; h < (chunks > 1 ? 2 : 1); ++h) {
+    HIPCHECK(ctx->b_io[h].ensure(std::max<size_t>(off[h] + bytes, 65536)));
+    if (chunks > 1 && !ctx->b_ev[h]) HIPCHECK(hipEventCreateWithFlags(&ctx->b_ev[h], hipEventDisableTiming));
+  }
+  if (!tables.empty()) std::memcpy(ctx->b_io[0].p, tables.data(), tables.size());
+  hipError_t e = hipSuccess;
+  for (long long c = 0; c <= chunks && e == hipSuccess; ++c) {
+    const int h = int(c & 1);
+    if (c < chunks) {
+      const long long first = c * kBatchChunk, count = std::min(kBatchChunk, n - first);
+      fill(static_cast<unsigned char*>(ctx->b_io[h].p) + off[h], first, count);
+      e = launch(static_cast<unsigned char*>(ctx->b_io[h].dev) + off[h], count, st);
+      if (e == hipSuccess && chunks > 1) e = hipEventRecord(ctx->b_ev[h], st);
+    }
+    if (c > 0 && e == hipSuccess) {
+      const long long first = (c - 1) * kBatchChunk;
+      e = chunks > 1 ? hipEventSynchronize(ctx->b_ev[h ^ 1]) : hipStreamSynchronize(st);
+      if (e == hipSuccess)
+        drain(static_cast<unsigned char*>(ctx->b_io[h ^ 1].p) + off[h ^ 1], first, std::min(kBatchChunk, n - first));
+    }
+  }
+  if (e != hipSuccess) (void)hipStreamSynchronize(st);  // nothing may still use the chunks
+  HIPCHECK(e);
+  return MT_OK;
+}
 
 extern "C" {
 
@@ -1827,17 +1878,25 @@ int mt_stopping_batch_arith(mt_ctx* ctx, int arith, int Z1, double m1, int mat, 
   std::vector<unsigned char> blob;
   msg = build_tables(ctx->coef, ctx->tgt, species, blob);
   if (!msg.empty()) return fail(MT_E_LIMIT, msg);
-  hipStream_t st = ctx->stream;
-  HIPCHECK(ctx->tables.ensure(blob.size()));
-  HIPCHECK(ctx->scratch_a.ensure(n * sizeof(double)));
-  HIPCHECK(ctx->scratch_b.ensure(n * sizeof(double)));
-  HIPCHECK(hipMemcpyAsync(ctx->tables.p, blob.data(), blob.size(), hipMemcpyHostToDevice, st));
-  HIPCHECK(hipMemcpyAsync(ctx->scratch_a.p, E, n * sizeof(double), hipMemcpyHostToDevice, st));
-  HIPCHECK(stopping_launch(arith, ctx->tables.as<unsigned char>(), ps[0], mat, ctx->scratch_a.as<double>(), n,
-                           ctx->scratch_b.as<double>(), st));
-  HIPCHECK(hipMemcpyAsync(se_out, ctx->scratch_b.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipStreamSynchronize(st));
-  return MT_OK;
+  // tables of up to 32 KB go to each block's LDS, larger ones to device memory
+  const bool in_lds = blob.size() <= 32768;
+  const int lds_bytes = in_lds ? int(blob.size()) : 0;
+  if (!in_lds) {
+    HIPCHECK(ctx->tables.ensure(blob.size()));
+    HIPCHECK(hipMemcpy(ctx->tables.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
+    blob.clear();
+  }
+  return run_batch(
+      ctx, n, 2 * sizeof(double), blob,
+      [&](unsigned char* h, long long first, long long cnt) { std::memcpy(h, E + first, cnt * sizeof(double)); },
+      [&](unsigned char* d, long long cnt, hipStream_t st) {
+        double* e = reinterpret_cast<double*>(d);
+        const unsigned char* tab = in_lds ? static_cast<unsigned char*>(ctx->b_io[0].dev) : ctx->tables.as<unsigned char>();
+        return stopping_launch(arith, tab, lds_bytes, ps[0], mat, e, cnt, e + cnt, st);
+      },
+      [&](unsigned char* h, long long first, long long cnt) {
+        std::memcpy(se_out + first, reinterpret_cast<double*>(h) + cnt, cnt * sizeof(double));
+      });
 }
 
 int mt_stopping_batch(mt_ctx* ctx, int Z1, double m1, int mat, const double* E, long long n, double* se_out) {
@@ -1854,18 +1913,6 @@ int mt_scatter_batch_arith(mt_ctx* ctx, int arith, int potential, const double* 
   if (arith == MT_FP32_SURROGATE && !ctx->mlp_ready) return fail(MT_E_STATE, "no surrogate installed");
   if (n <= 0) return MT_OK;
   HIPCHECK(hipSetDevice(ctx->device));
-  hipStream_t st = ctx->stream;
-  HIPCHECK(ctx->scratch_a.ensure(n * sizeof(double)));
-  HIPCHECK(ctx->scratch_b.ensure(n * sizeof(double)));
-  HIPCHECK(ctx->scratch_c.ensure(n * sizeof(double)));
-  HIPCHECK(ctx->scratch_d.ensure(n * sizeof(double)));
-  HIPCHECK(ctx->scratch_e.ensure(n * 2 * sizeof(double)));
-  HIPCHECK(hipMemcpyAsync(ctx->scratch_a.p, eps, n * sizeof(double), hipMemcpyHostToDevice, st));
-  HIPCHECK(hipMemcpyAsync(ctx->scratch_b.p, b, n * sizeof(double), hipMemcpyHostToDevice, st));
-  double* d_s2 = ctx->scratch_c.as<double>();
-  double* d_ct = ctx->scratch_d.as<double>();
-  double* d_st = ctx->scratch_e.as<double>();
-  int* d_it = reinterpret_cast<int*>(d_st + n);
   MlpDev S;
   std::memset(&S, 0, sizeof(S));
   if (arith == MT_FP32_SURROGATE) {
@@ -1874,14 +1921,24 @@ int mt_scatter_batch_arith(mt_ctx* ctx, int arith, int potential, const double* 
     S.n = ctx->mlp_norm;
     S.bf16 = ctx->mlp_bf16;
   }
-  HIPCHECK(scatter_launch(arith, potential, S, ctx->scratch_a.as<double>(), ctx->scratch_b.as<double>(), n, d_s2,
-                          d_ct, d_st, d_it, st));
-  HIPCHECK(hipMemcpyAsync(s2, d_s2, n * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipMemcpyAsync(ct, d_ct, n * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipMemcpyAsync(st_out, d_st, n * sizeof(double), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipMemcpyAsync(iters, d_it, n * sizeof(int), hipMemcpyDeviceToHost, st));
-  HIPCHECK(hipStreamSynchronize(st));
-  return MT_OK;
+  return run_batch(
+      ctx, n, 5 * sizeof(double) + sizeof(int), {},
+      [&](unsigned char* h, long long first, long long cnt) {
+        std::memcpy(h, eps + first, cnt * sizeof(double));
+        std::memcpy(h + cnt * sizeof(double), b + first, cnt * sizeof(double));
+      },
+      [&](unsigned char* d, long long cnt, hipStream_t st) {
+        double* x = reinterpret_cast<double*>(d);
+        return scatter_launch(arith, potential, S, x, x + cnt, cnt, x + 2 * cnt, x + 3 * cnt, x + 4 * cnt,
+                              reinterpret_cast<int*>(x + 5 * cnt), st);
+      },
+      [&](unsigned char* h, long long first, long long cnt) {
+        const double* x = reinterpret_cast<const double*>(h);
+        std::memcpy(s2 + first, x + 2 * cnt, cnt * sizeof(double));
+        std::memcpy(ct + first, x + 3 * cnt, cnt * sizeof(double));
+        std::memcpy(st_out + first, x + 4 * cnt, cnt * sizeof(double));
+        std::memcpy(iters + first, x + 5 * cnt, cnt * sizeof(int));
+      });
 }
 
 int mt_scatter_batch(mt_ctx* ctx, int potential, const double* eps, const double* b, long long n, double* s2,
