@@ -126,7 +126,7 @@ struct Params {
   // work distribution
   unsigned long long* ctrl;
   Queue q;
-  double half_share;            // 1 / (2 waves)
+  double even_share;            // 1 / waves
   // a small batch (at most 64 primaries per SIMD): primaries a wave admits at
   // once, without the budget (0: not small), and the first block to start late
   // (0: none)

@@ -422,7 +422,8 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
         // of it: the longest chains start at once, on every SIMD (64 a wave
         // left most waves to the queue: 2000 He histories 8.5 -> 4.4 ms).
         // Else what the cascade budget leaves (see Params), except a wave's
-        // first, which all waves make before a cascade has ended.
+        // first, which all waves make before a cascade has ended (with roles
+        // the feeders would flood the queue: 2e5 He histories 47 against 29 ms).
         auto may_admit = [&](int most) -> long long {
           if (A->admit_share > 0) return min(most, A->admit_share);
           const uint64_t live = ld_relaxed(&ctrl[kLive]);
@@ -432,7 +433,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           const long long cmax = max((long long)(A->budget / fmax(fhat, 1.0)), A->c_floor);
           const long long n = min((long long)most, cmax - (long long)live);
           if (!A->admit_strict) {
-            if (!first_adm) return n;
+            if (!first_adm || roles) return n;
             first_adm = false;
             return most;
           }
@@ -466,11 +467,15 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
         const bool may_pop = t0 > h0;
         // a wave that is not feeding admits primaries when the queue has
         // nothing for it: as many as it has idle lanes, and without roles up
-        // to `want` while that is less than half an even share of those left
-        // (the last ones are spread over the waves)
+        // to `want` while that is less than an even share of those left (the
+        // last ones are spread over the waves).  Of half a share a wave polls
+        // too often where a history is short (3e5 wire histories: 64 at a time
+        // 10.2 ms, half a share 10.7, one 10.0); 64 at a time leaves the last
+        // ones to a few waves (2e5 He histories: 33.4, 22.6, 23.5 ms; 1e5 C
+        // histories in W: 85, 56, 58 ms).
         if (!feeding && !may_pop && pka_left > 0) {
           const int need = n_idle - scount;
-          const long long even = roles ? 0ll : (long long)((double)pka_left * A->half_share);
+          const long long even = roles ? 0ll : (long long)((double)pka_left * A->even_share);
           n_adm = may_admit(min(want, max(need, (int)min(even, 64ll))));
         }
         const bool may_pka = n_adm > 0;
