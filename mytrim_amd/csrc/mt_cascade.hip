@@ -222,7 +222,7 @@ __device__ __forceinline__ void physics(const TableView& T, int sp, int k, doubl
     // impact parameter and target atom (trim.C:143-160)
     const double p = pmax * m_sqrt(u53(blk.x, blk.y));
     eps = ec.fi * E;
-    const double b = p * ec.inv_ai;
+    const double b = p * ec.ai;  // the reciprocal, in this kernel's copy
     // electronic loss along ls (trim.C:166-170) and scattering (trim.C:172-272)
     dee = ls * getrstop<double>(T, sp, k, E, lE);
     scatter<double, POT>(eps, b, lE + ec.ln_fi, s2, ct, st, it);
@@ -286,12 +286,12 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   // queue on the word's cache line
   if (threadIdx.x == 0 && atomicAdd(&P.ctrl[kState], (unsigned long long)nwb << 16) == ~0ull) err |= kErrBadEntry;
   __syncthreads();
-  {  // reciprocals the collisions share, by the arithmetic that they used for each
+  if constexpr (ARITH == 0) {  // reciprocals the collisions share, by the arithmetic that they used for each
     const TableHeader* h = (const TableHeader*)lds;
     ElemConst* el = (ElemConst*)(lds + h->off_el);
-    for (int i = threadIdx.x; i < h->n_species * h->n_el; i += blockDim.x) el[i].inv_ai = m_rcp(el[i].ai);
+    for (int i = threadIdx.x; i < h->n_species * h->n_el; i += blockDim.x) el[i].ai = m_rcp(el[i].ai);
+    __syncthreads();
   }
-  __syncthreads();
 
   const TableHeader* H = (const TableHeader*)lds;
   TableView T;

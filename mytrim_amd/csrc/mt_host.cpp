@@ -94,7 +94,7 @@ static StopConst make_stop(const std::vector<CoefRow>& coef, int z1, double m_io
       const double mid = 0.5 * (lo + hi);
       (vr(mid) < limit ? lo : hi) = mid;
     }
-    c.e_low = vr(0.0) < limit ? 25.0 * lo * lo * vfermi * vfermi * (1.0 - 1e-6) : 0.0;
+    c.e_low = vr(0.0) < limit ? float(25.0 * lo * lo * vfermi * vfermi * (1.0 - 1e-6)) : 0.0f;
   }
   c.bq = (std::min(0.43, std::max(0.32, 0.12 + 0.025 * fz1))) / c.cbrt_fz1;
   c.l0k = std::min(1.2, 0.6 + fz1 / 30.0);

@@ -26,9 +26,8 @@ struct MatConst {   // per (species, material)
 
 struct ElemConst {  // per (species, element)
   double t;         // normalised stoichiometric fraction
-  double fi, ai, ec, my;
+  double fi, ai, ec, my;  // the FP64 cascade kernel's copy (LDS) holds 1 / ai in ai
   double ln_fi;     // log fi: log eps = log E + ln_fi
-  double inv_ai;    // the kernel's own reciprocal of ai, set in its copy (LDS)
   double Edisp, Elbind;
   int Z;
   int recoil_species;
@@ -42,7 +41,6 @@ struct StopConst {  // per (species, element): rstop(ion, Z2)
   double cbrt_fz1, cbrt2_fz1;
   double yr_lo;                 // vrmin / cbrt2_fz1
   double yr_branch;             // max(yrmin, vrmin / cbrt2_fz1)
-  double e_low;                 // below this e (keV/amu) yr is yr_branch (0: nowhere)
   double vk;                    // 3 vfermi / 4
   double bq;                    // min(0.43, max(0.32, 0.12 + 0.025 Z1)) / cbrt(Z1)
   double l0k;                   // min(1.2, 0.6 + Z1/30)
@@ -59,8 +57,13 @@ struct StopConst {  // per (species, element): rstop(ion, Z2)
   double zeta_lo;               // heavy ions, low-velocity branch (yr = yr_branch): the
                                 // effective-charge factor before its z1^3 term
   int kind;                     // 1 proton, 2 helium, 3 heavy ion
-  int pad;
+  float e_low;                  // below this e (keV/amu) yr is yr_branch (0: nowhere)
 };
+
+// The tables share an LDS with the recoil stacks, so their size decides which
+// targets a launch shape takes: a double more in each of the two is 16 B times
+// species times elements (6 KB for a compound of 19 elements).
+static_assert(sizeof(ElemConst) == 72 && sizeof(StopConst) == 320, "constants per (species, element)");
 
 struct Species {
   int Z;

@@ -1,0 +1,36 @@
+"""Targets at the limit of a workgroup's LDS (160 KiB): tables, recoil stacks and
+what else a kernel keeps there."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from mytrim_amd import configs, gpu
+from mytrim_amd.problem import Element, Material
+
+pytestmark = pytest.mark.gpu
+
+
+def compound(n, n_hist):
+    """n elements in one material, the primary another species: the tables take
+    544 + (n + 1) (64 + 392 n) bytes, 150 784 for 19."""
+    els = [Element(Z, 2.0 * Z + 1.0, 1.0, 25.0, 3.0) for Z in range(20, 20 + n)]
+    return configs.vacancy_case("cu", 1e3, n_hist, seed=7).with_(materials=[Material(7.0, els)])
+
+
+# one wave per block, 80 B a stack entry: 150 784 + 8000 of 163 840
+@pytest.mark.parametrize("stack_cap", [100])
+def test_cascades_in_a_full_lds(stack_cap):
+    prob = compound(19, 200)
+    e = gpu.Engine(0)
+    try:
+        e.tune(block=64, blocks_per_cu=1, stack_cap=stack_cap)
+        r = e.run(prob)
+        e.tune(block=64, blocks_per_cu=1, stack_cap=64)
+        s = e.run(prob)
+        for k in ("n_coll", "n_flight", "vac", "repl", "subst", "inter"):
+            assert r[k] == s[k] > 0, k
+        assert np.array_equal(r["vac_hist"], s["vac_hist"])
+        o = O.run(prob, rng=1, nthreads=4)
+        assert r["n_flight"] == pytest.approx(o["n_flight"], rel=0.01)
+    finally:
+        e.close()
