@@ -281,35 +281,41 @@ struct mt_ctx {
   }
 };
 
-// A batch of n elements through the mapped chunks: `fill` copies elements
-// [first, first + count) in, `launch` runs the kernel on them, `drain` copies
-// the results out; a chunk's kernel runs while the other chunk is copied.  One
-// launch and one wait for a small batch: a table of 97 stopping powers takes
-// 22 us, with three copies around its kernel it took 36 us (launch and wait
-// alone are 11 us).  No page of the caller's arrays is pinned for a large one:
-// 250 001 deflections take 0.91 ms against 0.99 ms.  Chunks of 2^16: the copies
-// of one take as long as the kernel of the other.  A context's first batch also
-// pays for the pinned buffer (11 us for any size up to 256 KiB).
+// A batch of n elements: `fill` copies elements [first, first + count) in, `launch`
+// runs the kernel on them, `drain` copies the results out.  An element takes
+// bytes_each.  `tables`, if any, go along; `launch` gets their device address.
+// Through mapped chunks: one launch and one wait for a small batch (a table of 97
+// stopping powers takes 20 us, with three copies around its kernel 34 us; launch
+// and wait alone are 11 us), and a chunk's kernel runs while the other chunk is
+// copied.  No page of the caller's arrays is pinned for a large one: 250 001
+// deflections take 0.78 ms against 0.99 ms.  Chunks of 2^16: the copies of one
+// take as long as the kernel of the other.
 constexpr long long kBatchChunk = 1ll << 16;
+constexpr size_t kLdsTables = 32768;  // larger tables are read from device memory
 template <class Fill, class Launch, class Drain>
-static int run_batch(mt_ctx* ctx, long long n, size_t bytes_each, const std::vector<unsigned char>& tables, Fill fill,
-                     Launch launch, Drain drain) {
+static int run_batch(mt_ctx* ctx, long long n, size_t bytes_each, const std::vector<unsigned char>& tables, Fill fill, Launch launch, Drain drain) {
   hipStream_t st = ctx->stream;
+  const size_t off[2] = {(tables.size() + 255) & ~size_t(255), 0};  // where each buffer's chunk begins
   const long long chunks = (n + kBatchChunk - 1) / kBatchChunk;
   const size_t bytes = size_t(std::min(n, kBatchChunk)) * bytes_each;
-  const size_t off[2] = {(tables.size() + 255) & ~size_t(255), 0};  // where each buffer's chunk begins
   for (int h = 0; h < (chunks > 1 ? 2 : 1); ++h) {
     HIPCHECK(ctx->b_io[h].ensure(std::max<size_t>(off[h] + bytes, 65536)));
     if (chunks > 1 && !ctx->b_ev[h]) HIPCHECK(hipEventCreateWithFlags(&ctx->b_ev[h], hipEventDisableTiming));
   }
-  if (!tables.empty()) std::memcpy(ctx->b_io[0].p, tables.data(), tables.size());
+  const unsigned char* tab = static_cast<unsigned char*>(ctx->b_io[0].dev);
   hipError_t e = hipSuccess;
+  if (!tables.empty()) std::memcpy(ctx->b_io[0].p, tables.data(), tables.size());
+  if (tables.size() > kLdsTables) {  // from the pinned copy, in stream order
+    HIPCHECK(ctx->tables.ensure(tables.size()));
+    e = hipMemcpyAsync(ctx->tables.p, ctx->b_io[0].p, tables.size(), hipMemcpyHostToDevice, st);
+    tab = ctx->tables.as<unsigned char>();
+  }
   for (long long c = 0; c <= chunks && e == hipSuccess; ++c) {
     const int h = int(c & 1);
     if (c < chunks) {
       const long long first = c * kBatchChunk, count = std::min(kBatchChunk, n - first);
       fill(static_cast<unsigned char*>(ctx->b_io[h].p) + off[h], first, count);
-      e = launch(static_cast<unsigned char*>(ctx->b_io[h].dev) + off[h], count, st);
+      e = launch(static_cast<unsigned char*>(ctx->b_io[h].dev) + off[h], tab, count, st);
       if (e == hipSuccess && chunks > 1) e = hipEventRecord(ctx->b_ev[h], st);
     }
     if (c > 0 && e == hipSuccess) {
@@ -1882,20 +1888,12 @@ int mt_stopping_batch_arith(mt_ctx* ctx, int arith, int Z1, double m1, int mat, 
   std::vector<unsigned char> blob;
   msg = build_tables(ctx->coef, ctx->tgt, species, blob);
   if (!msg.empty()) return fail(MT_E_LIMIT, msg);
-  // tables of up to 32 KB go to each block's LDS, larger ones to device memory
-  const bool in_lds = blob.size() <= 32768;
-  const int lds_bytes = in_lds ? int(blob.size()) : 0;
-  if (!in_lds) {
-    HIPCHECK(ctx->tables.ensure(blob.size()));
-    HIPCHECK(hipMemcpy(ctx->tables.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
-    blob.clear();
-  }
+  const int lds_bytes = blob.size() <= kLdsTables ? int(blob.size()) : 0;
   return run_batch(
       ctx, n, 2 * sizeof(double), blob,
       [&](unsigned char* h, long long first, long long cnt) { std::memcpy(h, E + first, cnt * sizeof(double)); },
-      [&](unsigned char* d, long long cnt, hipStream_t st) {
+      [&](unsigned char* d, const unsigned char* tab, long long cnt, hipStream_t st) {
         double* e = reinterpret_cast<double*>(d);
-        const unsigned char* tab = in_lds ? static_cast<unsigned char*>(ctx->b_io[0].dev) : ctx->tables.as<unsigned char>();
         return stopping_launch(arith, tab, lds_bytes, ps[0], mat, e, cnt, e + cnt, st);
       },
       [&](unsigned char* h, long long first, long long cnt) {
@@ -1931,7 +1929,7 @@ int mt_scatter_batch_arith(mt_ctx* ctx, int arith, int potential, const double* 
         std::memcpy(h, eps + first, cnt * sizeof(double));
         std::memcpy(h + cnt * sizeof(double), b + first, cnt * sizeof(double));
       },
-      [&](unsigned char* d, long long cnt, hipStream_t st) {
+      [&](unsigned char* d, const unsigned char*, long long cnt, hipStream_t st) {
         double* x = reinterpret_cast<double*>(d);
         return scatter_launch(arith, potential, S, x, x + cnt, cnt, x + 2 * cnt, x + 3 * cnt, x + 4 * cnt,
                               reinterpret_cast<int*>(x + 5 * cnt), st);

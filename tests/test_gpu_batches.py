@@ -45,3 +45,26 @@ def test_tables_past_lds():
         assert np.max(np.abs(se - ref) / ref) < 1e-12
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("n_el", [2, 16])
+def test_repeated_calls_agree(n_el):
+    """A context's first small batches, its later ones and large ones take other
+    ways to the kernel; tables of 16 elements do not go to LDS."""
+    els = [Element(Z, 2.0 * Z + 1.0, 1.0, 25.0, 3.0) for Z in range(20, 20 + n_el)]
+    prob = configs.c2_cu_cu(1).with_(materials=[Material(7.0, els)])
+    E = np.geomspace(10.0, 1e7, 2 * CHUNK + 3)
+    e, whole = gpu.Engine(0), gpu.Engine(0)
+    try:
+        e.set_target(prob)
+        whole.set_target(prob)
+        ref = whole.stopping(54, 131.29, 0, E)
+        for n in (1, 2048, 2049, 2047, 97, CHUNK + 1, 5):
+            assert np.array_equal(e.stopping(54, 131.29, 0, E[:n]), ref[:n]), n
+            assert np.array_equal(e.stopping(54, 131.29, 0, E[-n:]), ref[-n:]), n
+        m = ref[::CHUNK]
+        exact = np.array([O.getrstop(54, 131.29, x, 7.0, [(el.Z, el.m, el.t) for el in els]) for x in E[::CHUNK]])
+        assert np.max(np.abs(m - exact) / exact) < 1e-12
+    finally:
+        e.close()
+        whole.close()
