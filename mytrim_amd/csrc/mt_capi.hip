@@ -244,6 +244,7 @@ struct mt_ctx {
   // for each
   MBuf b_io[2];
   hipEvent_t b_ev[2] = {nullptr, nullptr};
+  int b_copied = 0;  // batches that went through copies instead
   // scattering surrogate
   DBuf mlp_p, mlp_w2bf, mlp_X, mlp_T, mlp_rec, mlp_part, mlp_m, mlp_v, mlp_t, mlp_bl, mlp_tri;
   MlpNorm mlp_norm{};
@@ -283,19 +284,44 @@ struct mt_ctx {
 
 // A batch of n elements: `fill` copies elements [first, first + count) in, `launch`
 // runs the kernel on them, `drain` copies the results out.  An element takes
-// bytes_each.  `tables`, if any, go along; `launch` gets their device address.
+// bytes_each, its inputs (the first part of a chunk) bytes_in.  `tables`, if any,
+// go along; `launch` gets their device address.
 // Through mapped chunks: one launch and one wait for a small batch (a table of 97
 // stopping powers takes 20 us, with three copies around its kernel 34 us; launch
 // and wait alone are 11 us), and a chunk's kernel runs while the other chunk is
 // copied.  No page of the caller's arrays is pinned for a large one: 250 001
 // deflections take 0.78 ms against 0.99 ms.  Chunks of 2^16: the copies of one
 // take as long as the kernel of the other.
+// Pinning the chunks costs a context 33 us once, so its first kCopiedBatches
+// batches of up to kCopiedSize elements go through device memory and two copies
+// when the caller says that these are the cheaper ones (`copies`): a program that
+// asks for one table never pins.
 constexpr long long kBatchChunk = 1ll << 16;
+constexpr long long kCopiedSize = 2048;
+constexpr int kCopiedBatches = 2;
 constexpr size_t kLdsTables = 32768;  // larger tables are read from device memory
 template <class Fill, class Launch, class Drain>
-static int run_batch(mt_ctx* ctx, long long n, size_t bytes_each, const std::vector<unsigned char>& tables, Fill fill, Launch launch, Drain drain) {
+static int run_batch(mt_ctx* ctx, long long n, size_t bytes_each, size_t bytes_in, bool copies,
+                     const std::vector<unsigned char>& tables, Fill fill, Launch launch, Drain drain) {
   hipStream_t st = ctx->stream;
   const size_t off[2] = {(tables.size() + 255) & ~size_t(255), 0};  // where each buffer's chunk begins
+  if (copies && n <= kCopiedSize && !ctx->b_io[0].p && ctx->b_copied < kCopiedBatches) {
+    ++ctx->b_copied;
+    const size_t in = off[0] + size_t(n) * bytes_in, all = off[0] + size_t(n) * bytes_each;
+    std::vector<unsigned char> stage(all);
+    if (!tables.empty()) std::memcpy(stage.data(), tables.data(), tables.size());
+    fill(stage.data() + off[0], 0ll, n);
+    HIPCHECK(ctx->scratch_a.ensure(all));
+    unsigned char* d = ctx->scratch_a.as<unsigned char>();
+    hipError_t e = hipMemcpyAsync(d, stage.data(), in, hipMemcpyHostToDevice, st);
+    if (e == hipSuccess) e = launch(d + off[0], d, n, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(stage.data() + in, d + in, all - in, hipMemcpyDeviceToHost, st);
+    const hipError_t es = hipStreamSynchronize(st);  // on an error too: nothing may still use the stage
+    HIPCHECK(e);
+    HIPCHECK(es);
+    drain(stage.data() + off[0], 0ll, n);
+    return MT_OK;
+  }
   const long long chunks = (n + kBatchChunk - 1) / kBatchChunk;
   const size_t bytes = size_t(std::min(n, kBatchChunk)) * bytes_each;
   for (int h = 0; h < (chunks > 1 ? 2 : 1); ++h) {
@@ -1890,7 +1916,7 @@ int mt_stopping_batch_arith(mt_ctx* ctx, int arith, int Z1, double m1, int mat, 
   if (!msg.empty()) return fail(MT_E_LIMIT, msg);
   const int lds_bytes = blob.size() <= kLdsTables ? int(blob.size()) : 0;
   return run_batch(
-      ctx, n, 2 * sizeof(double), blob,
+      ctx, n, 2 * sizeof(double), sizeof(double), true, blob,
       [&](unsigned char* h, long long first, long long cnt) { std::memcpy(h, E + first, cnt * sizeof(double)); },
       [&](unsigned char* d, const unsigned char* tab, long long cnt, hipStream_t st) {
         double* e = reinterpret_cast<double*>(d);
@@ -1924,7 +1950,7 @@ int mt_scatter_batch_arith(mt_ctx* ctx, int arith, int potential, const double* 
     S.bf16 = ctx->mlp_bf16;
   }
   return run_batch(
-      ctx, n, 5 * sizeof(double) + sizeof(int), {},
+      ctx, n, 5 * sizeof(double) + sizeof(int), 2 * sizeof(double), false, {},
       [&](unsigned char* h, long long first, long long cnt) {
         std::memcpy(h, eps + first, cnt * sizeof(double));
         std::memcpy(h + cnt * sizeof(double), b + first, cnt * sizeof(double));
