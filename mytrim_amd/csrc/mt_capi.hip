@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <initializer_list>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -354,6 +355,23 @@ static int run_batch(mt_ctx* ctx, long long n, size_t bytes_each, size_t bytes_i
   if (e != hipSuccess) (void)hipStreamSynchronize(st);  // nothing may still use the chunks
   HIPCHECK(e);
   return MT_OK;
+}
+
+// A batch of several chunks writes results before it has read the last inputs:
+// inputs [in, in + n) that an output's bytes run into (at another place than its
+// own elements) are read from a copy.
+static const double* batch_input(const double* in, long long n, std::initializer_list<std::pair<const void*, size_t>> outs,
+                                 std::vector<double>& copy) {
+  if (n <= kBatchChunk) return in;
+  const uintptr_t a = uintptr_t(in), a_end = a + size_t(n) * sizeof(double);
+  for (const auto& o : outs) {
+    const uintptr_t b = uintptr_t(o.first), b_end = b + size_t(n) * o.second;
+    if (a != b && a < b_end && b < a_end) {
+      copy.assign(in, in + n);
+      return copy.data();
+    }
+  }
+  return in;
 }
 
 extern "C" {
@@ -1915,6 +1933,8 @@ int mt_stopping_batch_arith(mt_ctx* ctx, int arith, int Z1, double m1, int mat, 
   msg = build_tables(ctx->coef, ctx->tgt, species, blob);
   if (!msg.empty()) return fail(MT_E_LIMIT, msg);
   const int lds_bytes = blob.size() <= kLdsTables ? int(blob.size()) : 0;
+  std::vector<double> own;
+  E = batch_input(E, n, {{se_out, sizeof(double)}}, own);
   return run_batch(
       ctx, n, 2 * sizeof(double), sizeof(double), true, blob,
       [&](unsigned char* h, long long first, long long cnt) { std::memcpy(h, E + first, cnt * sizeof(double)); },
@@ -1949,6 +1969,11 @@ int mt_scatter_batch_arith(mt_ctx* ctx, int arith, int potential, const double* 
     S.n = ctx->mlp_norm;
     S.bf16 = ctx->mlp_bf16;
   }
+  std::vector<double> own_eps, own_b;
+  const std::initializer_list<std::pair<const void*, size_t>> outs = {
+      {s2, sizeof(double)}, {ct, sizeof(double)}, {st_out, sizeof(double)}, {iters, sizeof(int)}};
+  eps = batch_input(eps, n, outs, own_eps);
+  b = batch_input(b, n, outs, own_b);
   return run_batch(
       ctx, n, 5 * sizeof(double) + sizeof(int), 2 * sizeof(double), false, {},
       [&](unsigned char* h, long long first, long long cnt) {

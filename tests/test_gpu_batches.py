@@ -68,3 +68,27 @@ def test_repeated_calls_agree(n_el):
     finally:
         e.close()
         whole.close()
+
+
+def test_outputs_over_later_inputs():
+    """Results written over inputs that a later chunk reads, or over their own."""
+    n, shift = 3 * CHUNK + 5, CHUNK + 4321
+    rng = np.random.default_rng(3)
+    E = np.exp(rng.uniform(np.log(10.0), np.log(1e7), n))
+    eps, b = np.exp(rng.uniform(np.log(1e-4), np.log(30.0), n)), 8.0 * np.sqrt(1.0 - rng.random(n))
+    L, p = gpu.lib(), lambda a: a.ctypes.data_as(gpu.dp)
+    e = gpu.Engine(0)
+    try:
+        e.set_target(configs.c2_cu_cu(1))
+        se, sc = e.stopping(6, 12.011, 0, E), e.scatter(eps, b)
+        for s in (0, shift):
+            buf = np.concatenate([E, np.zeros(s)])
+            assert L.mt_stopping_batch(e.h, 6, 12.011, 0, p(buf), n, p(buf[s:])) == 0
+            assert np.array_equal(buf[s:s + n], se)
+            buf, bb = np.concatenate([eps, np.zeros(s)]), b.copy()
+            ct, st, it = np.zeros(n), np.zeros(n), np.zeros(n, np.int32)
+            assert L.mt_scatter_batch(e.h, 0, p(buf), p(bb), n, p(buf[s:]), p(ct), p(st), it.ctypes.data_as(gpu.ip)) == 0
+            for got, want in zip((buf[s:s + n], ct, st, it), sc):
+                assert np.array_equal(got, want)
+    finally:
+        e.close()
