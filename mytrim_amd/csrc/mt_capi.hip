@@ -813,11 +813,22 @@ static int run_shape(const mt_ctx* ctx, const mt_run_opts* o, size_t table_bytes
   s.block = ctx->tune.block ? ctx->tune.block : 256;
   s.cap = ctx->tune.stack_cap ? ctx->tune.stack_cap : 128;
   const int nwb = s.block / 64;
-  const size_t base = table_bytes + size_t(nwb) * cascade_stack_bytes(s.cap) + kNumEnergy * sizeof(double);
+  const size_t sums = kNumEnergy * sizeof(double);  // the block's rare energies
+  auto base_of = [&](int cap) { return table_bytes + size_t(nwb) * cascade_stack_bytes(cap) + sums; };
   const size_t lds_max = size_t(ctx->lds_max);
-  if (base > lds_max) return fail(MT_E_LIMIT, "tables and stacks exceed the LDS of a workgroup");
   const int arith = o->arith, pot = ctx->tgt.potential, geo = ctx->tgt.geo.kind;
   const int want = ctx->tune.blocks_per_cu > 0 ? ctx->tune.blocks_per_cu : kDefaultWavesPerCu * 64 / s.block;
+  // the sums are not to cost a shape its launch or a resident block: where they
+  // would, each stack gives up an entry (76 B) for them
+  if (s.cap > 1 && base_of(s.cap) - sums <= lds_max) {
+    int with = 0, without = 0;
+    if (base_of(s.cap) <= lds_max)
+      HIPCHECK(cascade_occupancy(arith, pot, geo, perhist, s.block, base_of(s.cap), &with));
+    if (with < want) HIPCHECK(cascade_occupancy(arith, pot, geo, perhist, s.block, base_of(s.cap) - sums, &without));
+    if (with < std::min(want, without)) --s.cap;
+  }
+  const size_t base = base_of(s.cap);
+  if (base > lds_max) return fail(MT_E_LIMIT, "tables and stacks exceed the LDS of a workgroup");
   // LDS bytes of nl bins of each histogram (16-byte multiples)
   auto hist_bytes = [](int nl) { return (2 * size_t(nl) * sizeof(uint32_t) + 15) & ~size_t(15); };
   int nl = ctx->tune.lds_hist < 0 ? 0 : o->vac_nb + 2;

@@ -12,21 +12,23 @@ pytestmark = pytest.mark.gpu
 
 def compound(n, n_hist):
     """n elements in one material, the primary another species: the tables take
-    544 + (n + 1) (64 + 392 n) bytes, 150 784 for 19."""
+    544 + (n + 1) (64 + 392 n) bytes: 72 784 for 13, 150 784 for 19."""
     els = [Element(Z, 2.0 * Z + 1.0, 1.0, 25.0, 3.0) for Z in range(20, 20 + n)]
     return configs.vacancy_case("cu", 1e3, n_hist, seed=7).with_(materials=[Material(7.0, els)])
 
 
-# one wave per block, 80 B a stack entry: 150 784 + 8000 of 163 840
-@pytest.mark.parametrize("stack_cap", [100])
-def test_cascades_in_a_full_lds(stack_cap):
-    prob = compound(19, 200)
+# one wave per block, 76 B a stack entry (rounded up to 16): 150 784 + 7600 of
+# 163 840; all but 48 B; half of the LDS but for 16 B, which takes two blocks
+@pytest.mark.parametrize("n_el,blocks,stack_cap", [(19, 1, 100), (19, 1, 171), (13, 2, 120)])
+def test_cascades_in_a_full_lds(n_el, blocks, stack_cap):
+    prob = compound(n_el, 200)
     e = gpu.Engine(0)
     try:
-        e.tune(block=64, blocks_per_cu=1, stack_cap=stack_cap)
+        e.tune(block=64, blocks_per_cu=blocks, stack_cap=stack_cap, lds_hist=-1)
         r = e.run(prob)
-        e.tune(block=64, blocks_per_cu=1, stack_cap=64)
+        e.tune(block=64, blocks_per_cu=1, stack_cap=64, lds_hist=-1)
         s = e.run(prob)
+        assert r["grid"] == blocks * s["grid"]
         for k in ("n_coll", "n_flight", "vac", "repl", "subst", "inter"):
             assert r[k] == s[k] > 0, k
         assert np.array_equal(r["vac_hist"], s["vac_hist"])
