@@ -29,6 +29,10 @@ struct FlightSlot {
   int nn, Z, need, redo;     // target element; draws ran out; wave 3 drew again (2: they ran out)
 };
 
+// bytes at the start of the tables that are not copied to LDS
+constexpr int kFlightSkip = int(sizeof(TableHeader) & ~size_t(15));
+static_assert(2 * sizeof(FlightSlot) <= kFlightSkip, "slots within the header's place");
+
 // A collision whose direction and event are still to be worked out
 struct FlightPending {
   double E, p1E, den, dee, ls, rE, ct, st, my;
@@ -58,27 +62,28 @@ struct FlightPending {
 template <int POT>
 __global__ void __launch_bounds__(256) flight_kernel(FlightParams P) {
   // the block copies the ion's tables to LDS; each collision then reads its
-  // constants there (about a hundred cycles) instead of from L2
+  // constants there (about a hundred cycles) instead of from L2.  The header
+  // stays behind: the slots take no more than its place, so that the tables
+  // alone decide which targets fit the LDS
   extern __shared__ __align__(16) unsigned char lds_tables[];
   __shared__ FlightSlot slots[2];
+  const TableHeader* H = (const TableHeader*)P.tables;
   {
-    const uint4* src = (const uint4*)P.tables;
+    const uint4* src = (const uint4*)(P.tables + kFlightSkip);
     uint4* dst = (uint4*)lds_tables;
-    for (int i = threadIdx.x; i < P.table_bytes / 16; i += blockDim.x) dst[i] = src[i];
+    for (int i = threadIdx.x; i < (P.table_bytes - kFlightSkip) / 16; i += blockDim.x) dst[i] = src[i];
   }
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const unsigned char* blob = lds_tables;
-  const TableHeader* H = (const TableHeader*)blob;
   TableView T;
   T.n_species = H->n_species;
   T.n_mat = H->n_mat;
   T.n_el = H->n_el;
   T.potential = H->potential;
-  T.mat = (const MatConst*)(blob + H->off_mat);
-  T.el = (const ElemConst*)(blob + H->off_el);
-  T.stop = (const StopConst*)(blob + H->off_stop);
+  T.mat = (const MatConst*)(lds_tables + (H->off_mat - kFlightSkip));
+  T.el = (const ElemConst*)(lds_tables + (H->off_el - kFlightSkip));
+  T.stop = (const StopConst*)(lds_tables + (H->off_stop - kFlightSkip));
   const Geometry& G = P.geo;
   // arguments used in every collision, held in vector registers (there are
   // plenty): read from the argument segment one by one they cost a merge some
@@ -344,7 +349,7 @@ __global__ void __launch_bounds__(256) flight_kernel(FlightParams P) {
 }
 
 hipError_t flight_launch(const FlightParams& P, int potential, hipStream_t stream) {
-  const unsigned lds = unsigned(P.table_bytes);
+  const unsigned lds = unsigned(P.table_bytes - kFlightSkip);
   if (potential == 1)
     hipLaunchKernelGGL(flight_kernel<1>, dim3(1), dim3(256), lds, stream, P);
   else if (potential == 2)
