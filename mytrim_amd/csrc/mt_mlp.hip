@@ -78,8 +78,9 @@ __global__ void __launch_bounds__(256) mlp_data(uint32_t seed, long long n, cons
 // mlp_pass: forward and backward pass of 16 samples per block (256 blocks for a
 // batch of 4096): z2 = h1 W2^T, y = h2 W3, g1 = d2 W2, a wave per 16 columns.
 // The activations and deltas go to `rec` ([h1 | d1 | h2 | d2][S][64], then dy[S]
-// and e^2[S], S the batch rounded up to whole chunks, then 1 and 0; deltas of the
-// samples past the batch are zero).
+// and e^2[S], S the batch rounded up to whole chunks, then 1 and 0; activations and
+// deltas of the samples past the batch are zero, whatever the weights: 0 times an
+// infinite one would reach the sums).
 // mlp_grad: sums of delta x input over a chunk of 128 samples, a wave per 16 x 16
 // tile of a weight matrix, into part[chunk][kMlpParams + 1] (the last entry: the
 // squared errors).
@@ -130,7 +131,8 @@ __global__ void __launch_bounds__(256) mlp_pass(const float* __restrict__ p, con
 #pragma unroll
   for (int r = 0; r < 4; ++r) {  // layer 1 (mlp_h1): unit l of samples 4 w + r
     const int sm = 4 * w + r;
-    const float h = mlp_tanh(f[0] * xs[0][sm] + f[1] * xs[1][sm] + f[2] * xs[2][sm] + f[3]);
+    const float t1 = mlp_tanh(f[0] * xs[0][sm] + f[1] * xs[1][sm] + f[2] * xs[2][sm] + f[3]);
+    const float h = s0 + sm < B ? t1 : 0.0f;
     h1[sm * kHs + l] = h;
     rh1[(size_t)(s0 + sm) * kMlpH + l] = h;
   }
@@ -142,7 +144,7 @@ __global__ void __launch_bounds__(256) mlp_pass(const float* __restrict__ p, con
   float h2r[4];
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    h2r[r] = mlp_tanh(z[r]);
+    h2r[r] = s0 + 4 * q + r < B ? mlp_tanh(z[r]) : 0.0f;
     h2[(4 * q + r) * kHs + col] = h2r[r];
     rh2[(size_t)(s0 + 4 * q + r) * kMlpH + col] = h2r[r];
   }
@@ -167,7 +169,7 @@ __global__ void __launch_bounds__(256) mlp_pass(const float* __restrict__ p, con
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float d = dys[4 * q + r] * w3 * (1.0f - h2r[r] * h2r[r]);
+    const float d = s0 + 4 * q + r < B ? dys[4 * q + r] * w3 * (1.0f - h2r[r] * h2r[r]) : 0.0f;
     d2[(4 * q + r) * kHs + col] = d;
     rd2[(size_t)(s0 + 4 * q + r) * kMlpH + col] = d;
   }
@@ -179,7 +181,7 @@ __global__ void __launch_bounds__(256) mlp_pass(const float* __restrict__ p, con
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const float h = h1[(4 * q + r) * kHs + col];
-    rd1[(size_t)(s0 + 4 * q + r) * kMlpH + col] = g[r] * (1.0f - h * h);
+    rd1[(size_t)(s0 + 4 * q + r) * kMlpH + col] = s0 + 4 * q + r < B ? g[r] * (1.0f - h * h) : 0.0f;
   }
 }
 

@@ -31,3 +31,34 @@ def test_gradient_chunks(n):
         assert np.array_equal(g, again)
     finally:
         e.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 17, 128, 129])
+def test_gradient_with_infinite_weights(n):
+    """A unit with an infinite weight is saturated: its gradient is zero, the others
+    are finite, and the places of the last tile past the batch add nothing."""
+    prob = configs.c5_c_w(10, seed=43)
+    e = gpu.Engine(0)
+    try:
+        e.set_target(prob)
+        opts = gpu.Engine.surrogate_opts(prob)
+        norm = e.surrogate_norm(opts)
+        rng = np.random.default_rng(n)
+        p = gpu.Engine.surrogate_init(n)
+        p[3 * 5] = np.inf    # W1: unit 5, log eps
+        p[256 + 64 * 7 + 5] = -np.inf  # W2: unit 7, from unit 5
+        eps = np.exp(rng.uniform(np.log(norm["eps_lo"]), np.log(norm["eps_hi"]), n))
+        b = norm["b_hi"] * np.sqrt(rng.random(n))
+        ls2 = -8.0 + 8.0 * rng.uniform(-1.0, 1.0, n)
+        g, loss = e.surrogate_grad(opts, p, eps, b, ls2)
+        # 0 times the infinite weight, in the delta of unit 5, is not a number in
+        # the reference either: its own row of W1 and its bias
+        with np.errstate(invalid="ignore"):
+            ref_loss, ref = M.loss_grad(p, M.inputs(norm, eps, b), M.target(norm, ls2))
+        assert np.array_equal(np.isfinite(g), np.isfinite(ref)) and np.isfinite(g).sum() > 4400
+        ok = np.isfinite(ref)
+        assert np.linalg.norm((g - ref)[ok]) <= 3e-6 * np.linalg.norm(ref[ok]) + 1e-9
+        assert loss == pytest.approx(ref_loss, rel=3e-6)
+    finally:
+        e.close()
