@@ -741,8 +741,6 @@ static_assert(sizeof(LogRecord) == sizeof(mt_record) && sizeof(mt_record) == 80,
 // ------------------------------------------------------------ run pieces
 // (shared by mt_run_cascades, mt_run_cascades_log and mt_run_cascades_noalloc)
 
-constexpr uint64_t kMaxQueue = uint64_t(1) << 27;  // most queue slots a run takes by itself
-
 // bytes per slot of each queue array (px py pz dx dy dz E key mt: 8, hist: 4, ready: 8)
 constexpr size_t kQueueFieldBytes[kQueueArrays] = {8, 8, 8, 8, 8, 8, 8, 8, 8, 4, 8};
 
@@ -764,9 +762,9 @@ static int validate_run(const mt_ctx* ctx, const mt_primaries* pk, const mt_run_
 // what a run needs of its primaries besides their arrays
 struct PrimaryStats {
   double E0 = 0.0;  // total energy
-  int n = 0;        // species, each with its largest energy
+  int n = 0;        // species, each with its number, total and largest energy
   int Z[kMaxSpecies];
-  double m[kMaxSpecies], e_max[kMaxSpecies];
+  double m[kMaxSpecies], num[kMaxSpecies], e_sum[kMaxSpecies], e_max[kMaxSpecies];
 };
 
 // finite positive energies and positions, non-zero directions; the batch's
@@ -787,12 +785,20 @@ static int check_primaries(const mt_primaries* pk, PrimaryStats& st) {
     if (s == st.n && st.n < kMaxSpecies) {
       st.Z[s] = pk->Z[i];
       st.m[s] = pk->m[i];
-      st.e_max[s] = 0.0;
+      st.num[s] = st.e_sum[s] = st.e_max[s] = 0.0;
       ++st.n;
     }
-    if (s < st.n) st.e_max[s] = std::max(st.e_max[s], pk->E[i]);
+    if (s < st.n) {
+      st.num[s] += 1.0;
+      st.e_sum[s] += pk->E[i];
+      st.e_max[s] = std::max(st.e_max[s], pk->E[i]);
+    }
   }
-  if (pk->pka_uniform) st.E0 = pk->E[0] * double(pk->n_hist);
+  if (pk->pka_uniform) {
+    st.E0 = pk->E[0] * double(pk->n_hist);
+    st.num[0] = double(pk->n_hist);
+    st.e_sum[0] = st.E0;
+  }
   return MT_OK;
 }
 
@@ -880,6 +886,29 @@ static double flights_per_cascade0(const mt_ctx* ctx, const PrimaryStats& st, co
   return f;
 }
 
+// what the batch brings; the direct recoils only where its flights do not fit the
+// queue (an estimate per species and material, some 5 us each)
+static BatchWork batch_work(const mt_ctx* ctx, const PrimaryStats& st, const mt_run_opts* o, long long n, double flights,
+                            uint64_t qcap) {
+  BatchWork b;
+  b.n = n;
+  b.flights = flights;
+  if (double(n) * flights <= 2.0 * double(qcap) || o->follow_max_gen == 0 || o->follow_max_gen == 1) return b;
+  double ed_min = 1e300;
+  for (const HostMaterial& m : ctx->tgt.mat)
+    for (const HostElement& e : m.el) ed_min = std::min(ed_min, e.Edisp);
+  for (int s = 0; s < st.n; ++s) {
+    double mean = 0.0, most = 0.0;
+    for (const HostMaterial& m : ctx->tgt.mat) {
+      mean = std::max(mean, direct_estimate(st.Z[s], st.m[s], st.e_sum[s] / st.num[s], m.az, m.am, ed_min));
+      most = std::max(most, direct_estimate(st.Z[s], st.m[s], st.e_max[s], m.az, m.am, ed_min));
+    }
+    b.direct_all += st.num[s] * mean;
+    b.direct_max = std::max(b.direct_max, most);
+  }
+  return b;
+}
+
 // device memory of one run
 struct RunMem {
   const unsigned char* tables = nullptr;
@@ -897,7 +926,7 @@ struct RunMem {
 // the kernel parameters every run shares (per-history arrays, event streams
 // and the surrogate are set by the caller)
 static void fill_params(Params& P, const mt_ctx* ctx, const mt_primaries* pk, const mt_run_opts* o,
-                        const RunMem& M, const RunShape& sh, double f_init, const size_t* hoff) {
+                        const RunMem& M, const RunShape& sh, const BatchWork& work, const size_t* hoff) {
   std::memset(&P, 0, sizeof(P));
   P.tables = M.tables;
   P.table_bytes = M.table_bytes;
@@ -940,23 +969,15 @@ static void fill_params(Params& P, const mt_ctx* ctx, const mt_primaries* pk, co
   Q.nq = nq;
   Q.sub_log2 = log2cap - lq;
   Q.sub_mask = (uint64_t(1) << Q.sub_log2) - 1;
-  // a queue smaller than the batch's expected flights needs the budget kept;
-  // one wave per SIMD of a small batch admits all of it
-  const int first = std::min(sh.waves, 4 * ctx->cus);
   P.even_share = 1.0 / sh.waves;
-  const bool roomy = double(pk->n_hist) * f_init <= 2.0 * double(M.qcap);
-  P.admit_strict = !roomy && M.qcap < kMaxQueue;
-  if (ctx->tune.primary_waves64 == 0 && !P.admit_strict && pk->n_hist <= 64ll * first) {
-    P.admit_share = int((pk->n_hist + first - 1) / first);
-    P.late_block = sh.waves > first ? first * 64 / sh.block : 0;
-  }
-  // With wave roles, a batch of which the feeders' first admission takes nearly
-  // all is not held back for the rest: feeders that wait for the budget poll
-  // four words that every wave writes (2e5 He histories: 47 against 29 ms).
-  const bool all_at_once = ctx->tune.primary_waves64 > 0 && pk->n_hist <= 128ll * sh.waves;
-  P.budget = P.admit_strict ? 12.0 * double(M.qcap) + 1024.0 * sh.waves : (all_at_once ? 4.0 : 0.5) * double(M.qcap);
-  P.f_init = f_init;
-  P.c_floor = P.admit_strict ? std::min(512, sh.waves) : sh.waves;
+  const AdmitPlan plan = plan_admission(work, M.qcap, sh.waves, 4 * ctx->cus, sh.block, sh.cap, ctx->tune.primary_waves64);
+  P.admit_strict = plan.strict;
+  P.admit_share = plan.share;
+  P.late_block = plan.late_block;
+  P.budget = plan.budget;
+  P.f_init = work.flights;
+  P.c_floor = plan.live_floor;
+  P.c_cap = (long long)std::max(plan.live_cap, double(plan.live_floor));
   P.h_out = M.h_out;
   P.max_ic = 10000000;
   P.max_wait_ticks = (unsigned long long)(60.0 * ctx->clock_khz * 1000.0);
@@ -1132,7 +1153,7 @@ static int run_cascades(mt_ctx* ctx, const mt_primaries* pk, const mt_run_opts* 
   M.wave_energy = ctx->wave_energy.as<double>();
   M.h_out = ctx->h_out.as<int>();
   Params P;
-  fill_params(P, ctx, pk, o, M, sh, f_init, hoff);
+  fill_params(P, ctx, pk, o, M, sh, batch_work(ctx, ps, o, pk->n_hist, f_init, M.qcap), hoff);
   unsigned long long* res = M.res;
   if (perhist) {
     P.h_vac = ctx->per[0].as<int>();
@@ -1902,7 +1923,7 @@ int mt_run_cascades_noalloc(mt_ctx* ctx, const mt_primaries* pk, const mt_run_op
   span(M.wave_energy, size_t(sh.waves) * 2 * kNumEnergy * sizeof(double));
   span(M.h_out, size_t(std::max<long long>(pk->n_hist, 1)) * sizeof(int));
   Params P;
-  fill_params(P, ctx, pk, o, M, sh, f_init, hoff);
+  fill_params(P, ctx, pk, o, M, sh, batch_work(ctx, ps, o, pk->n_hist, f_init, M.qcap), hoff);
   double* red = reinterpret_cast<double*>(M.res + kResReduced);
   HIPCHECK(zero_spans_launch(zs, st));
   HIPCHECK(hipEventRecord(ctx->ev0, st));

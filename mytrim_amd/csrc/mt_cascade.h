@@ -131,17 +131,15 @@ struct Params {
   // once, without the budget (0: not small), and the first block to start late
   // (0: none)
   int admit_share, late_block;
-  int admit_strict;             // small queue: the budget is reserved before it is used
+  int admit_strict;             // the budget is reserved before it is used
   // cascade budget: admitted-but-incomplete cascades times the flights per
   // cascade (f_init until 64 cascades completed, then flights ended per
-  // completed cascade, an overestimate) stays below `budget`; at least c_floor
-  // cascades may always be live.  A queue sized for the batch is budgeted half
-  // its entries, unreserved.  In one that was given (a fixed scratch, a
-  // tuning) and is smaller, some 3 % of a live cascade's flights wait, after
-  // the lanes and stacks hold theirs: 12 times its entries and 16 a lane, each
-  // cascade reserved before it starts (admit_strict).
+  // completed cascade, an overestimate) stays below `budget`; c_floor cascades
+  // may always be live, c_cap at most.  A queue that has room for what starts at
+  // once is budgeted half its entries, unreserved; else each cascade is reserved
+  // before it starts (admit_strict; plan_admission in mt_tune.h)
   double budget, f_init;
-  long long c_floor;
+  long long c_floor, c_cap;
   int* h_out;                   // per history: flights queued or running
   int primary_waves64;          // waves per 64 that feed primaries (0: all waves do everything)
   long long max_ic;             // collisions per flight before kErrRunaway

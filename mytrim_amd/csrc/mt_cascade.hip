@@ -14,9 +14,8 @@
 //     its fields are stored and loaded at agent scope and a ready word
 //     (lap << 32 | checksum of the fields) tells a reader that all of them
 //     have landed
-//   * primaries are claimed in wave batches from a counter under a cascade
-//     budget: live cascades x expected flights per cascade stay within half
-//     the queue capacity
+//   * primaries are claimed in wave batches from a counter; where what starts
+//     at once could fill the queue, under a cascade budget (plan_admission)
 //   * termination: a wave that finds no work registers idle in a packed
 //     (epoch | live | idle) word; every wave leaves once all live waves are
 //     idle, every shard is empty and the primaries are used up, observed
@@ -430,7 +429,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           const uint64_t done = ld_relaxed(&ctrl[kCascDone]);
           const double fhat =
               done >= 64ull ? (double)ld_relaxed(&ctrl[kFlightsEnded]) / (double)done : A->f_init;
-          const long long cmax = max((long long)(A->budget / fmax(fhat, 1.0)), A->c_floor);
+          const long long cmax = min(max((long long)(A->budget / fmax(fhat, 1.0)), A->c_floor), A->c_cap);
           const long long n = min((long long)most, cmax - (long long)live);
           if (!A->admit_strict) {
             if (!first_adm || roles) return n;

@@ -1,6 +1,7 @@
-// The flights a cascade is expected to have, and the launch phases of a cascade
-// launch with the rate they project for a launch of more histories (host code
-// of the runs and of the autotuner, mt_autotune).
+// The flights and direct recoils a cascade is expected to have, how a launch
+// admits its primaries, and the launch phases of a cascade launch with the rate
+// they project for a launch of more histories (host code of the runs and of the
+// autotuner, mt_autotune).
 //
 // A launch ramps up until the admission of its middle primary, runs at a
 // steady rate until the admission of its last one, then drains: the last
@@ -10,6 +11,8 @@
 // and the collisions done in them) plus the rest of its collisions at the
 // steady rate.
 #pragma once
+#include <stdint.h>
+
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -33,6 +36,110 @@ inline double flights_estimate(double Z1, double m1, double E, double Z2, double
                    (std::pow(z, 0.75) * std::pow(m1, 1.5) * std::sqrt(m2));
   const double g = eps + 0.40244 * std::pow(eps, 0.75) + 3.4008 * std::pow(eps, 1.0 / 6.0);
   return 1.0 + E / (1.0 + k * g) / std::max(Ed, 1.0);
+}
+
+// Direct recoils of that ion above Ed: collisions that transfer more than Ed, over
+// the stopping, by the Thomas-Fermi cross-section of Winterbon, Sigmund and
+// Sanders, d sigma = pi a^2 f(sqrt t) / (2 t^1.5) dt with f(x) = 1.309 x^(1/3) /
+// (1 + (2.618 x^(4/3))^(2/3))^1.5, and Lindhard's k sqrt(eps), for heavy ions
+// falling off as 1 / sqrt(eps) above 25 keV/amu Z1^(4/3).  0.9 to 1.9 times what
+// cascades have (H to U, 1 keV to 1 GeV); the integrals run on a grid of 64 steps in
+// log eps.
+inline double direct_estimate(double Z1, double m1, double E, double Z2, double m2, double Ed) {
+  constexpr int N = 64;
+  const double z = std::pow(Z1, 2.0 / 3.0) + std::pow(Z2, 2.0 / 3.0);
+  const double a = 0.8853 * 0.5292 / std::sqrt(z);
+  const double per_eV = a * m2 / (Z1 * Z2 * 14.4 * (m1 + m2));
+  const double gamma = 4.0 * m1 * m2 / ((m1 + m2) * (m1 + m2));
+  const double k = 0.0793 * std::pow(Z1, 2.0 / 3.0) * std::sqrt(Z2) * std::pow(m1 + m2, 1.5) /
+                   (std::pow(z, 0.75) * std::pow(m1, 1.5) * std::sqrt(m2));
+  const double e0 = per_eV * std::max(Ed, 1.0) / gamma, e1 = per_eV * E;  // eps of threshold and ion
+  if (!(e1 > e0)) return 0.0;
+  const double step = std::log(e1 / e0) / N, fast = Z1 > 2.0 ? 2.5e4 * m1 * std::pow(Z1, 4.0 / 3.0) : 1e300;
+  double over[N + 1];  // integral of f / x^2 from e0, x = sqrt t
+  double loss = 0.0, sum = 0.0, f0 = 0.0, x0 = 0.0, y0 = 0.0;
+  for (int i = 0; i <= N; ++i) {
+    const double x = e0 * std::exp(step * i), c = std::cbrt(x);
+    const double d = 1.0 + 1.899 * std::pow(x, 8.0 / 9.0);
+    const double f = 1.309 * c / (d * std::sqrt(d));
+    over[i] = i == 0 ? 0.0 : over[i - 1] + 0.5 * step * (f0 / x0 + f / x);
+    loss = i == 0 ? 0.75 * x * f : loss + 0.5 * step * (f0 * x0 + f * x);  // integral of f from 0
+    // transfers from Ed (x = sqrt(e0 eps), halfway to e0 on this grid) to the largest
+    const double n = over[i] - 0.5 * (over[i / 2] + over[(i + 1) / 2]);
+    const double e = x / per_eV;
+    const double se = k * std::sqrt(x) * std::min(1.0, fast / e);
+    const double y = n / gamma / (loss / x + se) * x;
+    if (i > 0) sum += 0.5 * step * (y0 + y);
+    f0 = f;
+    x0 = x;
+    y0 = y;
+  }
+  return sum;
+}
+
+// What a batch is expected to bring: flights per cascade, direct recoils of all
+// its primaries and of the one with the most.
+struct BatchWork {
+  long long n = 0;
+  double flights = 1.0, direct_all = 0.0, direct_max = 0.0;
+};
+
+// How a launch admits its primaries (see Params)
+struct AdmitPlan {
+  bool strict = false;       // cascades reserved before they start
+  int share = 0;             // small batch: primaries a wave admits at once, without the budget
+  int late_block = 0;        // small batch: first block to start late (0: none)
+  double budget = 0.0;       // flights of live cascades
+  long long live_floor = 0;  // cascades that may always be live
+  double live_cap = 0.0;     // cascades that may be live at most
+};
+
+constexpr uint64_t kMaxQueue = uint64_t(1) << 27;  // most queue slots a run takes by itself
+
+// A queue that has room for the batch's flights needs no care; of one that has not
+// (capped at kMaxQueue, a fixed scratch, a tuning), the recoils that wait decide.
+// Measured, per live cascade (D: direct recoils):
+//  - light ions (He in Fe, 2 MeV C in W): 0.5 to 0.9 D, while most lanes hold
+//    primaries: they bring their recoils faster than lanes come free
+//  - heavy ions on fewer cascades than lanes, which widen the tree: 4.4 D (Cu 500
+//    keV) to 5.9 D (Xe 2 MeV in UO2) with a primary on every 16th lane, 1.8 to 3.6 D
+//    on every second one, 0.2 to 0.8 D on every lane; 3 to 10 % of the flights
+// So everything may start at once while 5, 3 and 1 times the estimate of D (1.1 to
+// 1.5 times the truth for these ions) of what starts fits the slots.
+// Else cascades are reserved first (strict) and bounded twice: by flights, 12 times
+// the slots and 16 a lane in a small queue (of which lanes and stacks hold the most:
+// 3 % wait), 7.5 times the slots in one that is large beside them (10 % wait); and
+// by D, nine tenths of the slots.  By flights alone, 65 536 histories of 2 MeV C in W
+// overflowed 2^21 slots (D is 17 % of their flights).
+inline AdmitPlan plan_admission(const BatchWork& b, uint64_t qcap, int waves, int simds, int block, int stack_cap,
+                                int feeders64) {
+  AdmitPlan p;
+  const double slots = double(qcap), n = double(b.n), lanes = 64.0 * waves;
+  const bool roomy = n * b.flights <= 2.0 * slots;
+  const double x = n / lanes;  // primaries per lane
+  const double widen = x < 0.5 ? 5.0 - 2.0 / 3.0 * std::log2(16.0 * std::max(x, 1.0 / 16.0))
+                               : std::max(1.0, 3.0 - 4.0 * (x - 0.5));
+  const bool at_once = widen * std::min(b.direct_all, lanes * b.direct_max) <= slots;
+  p.strict = !roomy && (qcap < kMaxQueue || !at_once);
+  const int first = std::min(waves, simds);  // one wave per SIMD of a small batch admits all of it
+  if (feeders64 == 0 && !p.strict && b.n <= 64ll * first) {
+    p.share = int((b.n + first - 1) / first);
+    p.late_block = waves > first ? first * 64 / block : 0;
+  }
+  // With wave roles, a batch of which the feeders' first admission takes nearly
+  // all is not held back for the rest: feeders that wait for the budget poll
+  // four words that every wave writes (2e5 He histories: 47 against 29 ms).
+  const bool feed_all = feeders64 > 0 && b.n <= 128ll * waves;
+  p.budget = (feed_all ? 4.0 : 0.5) * slots;
+  p.live_floor = waves;
+  p.live_cap = 1e18;
+  if (p.strict) {
+    p.budget = std::min(12.0 * slots + 1024.0 * waves, 7.5 * slots + 6144.0 * waves);
+    p.live_floor = std::min(512, waves);
+    const double d = std::min(b.direct_max, 2.0 * b.direct_all / std::max(n, 1.0));
+    p.live_cap = (0.9 * slots + 0.5 * stack_cap * waves) / std::max(d, 1.0);
+  }
+  return p;
 }
 
 struct LaunchPhases {
