@@ -62,3 +62,26 @@ def test_gradient_with_infinite_weights(n):
         assert loss == pytest.approx(ref_loss, rel=3e-6)
     finally:
         e.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,lr", [(1000, 4e-3), (5 * 1000 + 17, 1e-30)])
+def test_direct_and_replayed_epochs_agree(n, lr):
+    """One epoch is launched step by step, several replay a captured one: the same
+    first epoch, of one step, or of steps too small to move a weight."""
+    prob = configs.c5_c_w(10, seed=43)
+    out = {}
+    for epochs in (1, 2, 3):
+        e = gpu.Engine(0)
+        try:
+            e.set_target(prob)
+            o = gpu.Engine.surrogate_opts(prob, n_train=n, epochs=epochs, batch=1000, lr=lr, seed=5)
+            out[epochs] = e.surrogate_train(o, gpu.Engine.surrogate_init(2))
+        finally:
+            e.close()
+    first = [r[1][0] for r in out.values()]
+    assert np.isfinite(first).all() and first[0] == first[1] == first[2] > 0.0
+    if lr < 1e-20:
+        assert all(np.all(r[1] == first[0]) for r in out.values())
+        # a bias starts at zero and moves by at most a step's size, 15 times
+        assert all(np.max(np.abs(r[0] - out[1][0])) <= 1e-28 for r in out.values())
