@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "mt_cascade.h"
+#include "mt_counts.h"
 #include "mt_geometry.h"
 #include "mt_mlp.h"
 #include "mt_philox.h"
@@ -1064,11 +1065,14 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           // A reader on another XCD may end this flight as soon as it sees
           // the ready word, so the history's flight-count increment must be
           // performed first: the ready word depends on the returned count,
-          // which makes the store wait for the atomic.  A count below 1
-          // cannot happen (the pushing flight is outstanding); it would mean
-          // corrupt bookkeeping, and the run is aborted.  The fields need no
-          // ordering: the reader checks the checksum.
-          const bool sane = inc_old >= 1;
+          // which makes the store wait for the atomic.  A count below 1 while
+          // primaries are left to start means corrupt bookkeeping, and the run
+          // is aborted; once all have started, waves stop counting one by one
+          // (mt_counts.h).  Their counter is then read by an addition of zero,
+          // which sees the latest value.  The fields need no ordering: the
+          // reader checks the checksum.
+          bool sane = inc_old >= 1;
+          if (!sane) sane = count_possible(inc_old, atomicAdd(&ctrl[kPkaNext], 0ull), A->n_hist);
           if (!sane) err |= kErrBadEntry;
           st_agent(&A->q.ready[slot], ((uint64_t)(sane ? lap : 0u) << 32) | sum);
         }
