@@ -803,7 +803,10 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           lg_follow = lg_above && (P.follow_max_gen < 0 || F.gen + 1 < P.follow_max_gen);
         }
         // fate of recoil and ion (trim.C:357-411)
-        double enuc = 0.0;  // to nuclear losses, added where the branches meet
+        // to nuclear losses from the recoil, added where the branches meet; the
+        // ion's rest is a term of its own (the sum of the two would be rounded
+        // before the compensated addition)
+        double enuc = 0.0;
         if (lost) {
           state = 4;
           atomicAdd(&lsum[eElost], F.E);
@@ -848,13 +851,13 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           } else {
             // replacementCollision (trim.C:388-395)
             state = (H->species[F.sp].Z == ec.Z) ? 1 : 2;
-            enuc += F.E;
+            kadd(enuc_s, enuc_e, F.E);
           }
         } else {
           enuc = rE + ec.Elbind;
           if (F.E < C->Ef) {
             state = 3;
-            enuc += F.E;
+            kadd(enuc_s, enuc_e, F.E);
           }
         }
         kadd(enuc_s, enuc_e, enuc);
