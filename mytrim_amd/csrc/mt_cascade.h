@@ -131,6 +131,7 @@ struct Params {
   // once, without the budget (0: not small), and the first block to start late
   // (0: none)
   int admit_share, late_block;
+  int stagger;                  // otherwise: naps over which the blocks start
   int admit_strict;             // the budget is reserved before it is used
   // cascade budget: admitted-but-incomplete cascades times the flights per
   // cascade (f_init until 64 cascades completed, then flights ended per

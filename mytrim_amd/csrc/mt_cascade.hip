@@ -371,12 +371,10 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   // Staggered start.  In a small batch the second and third wave of a SIMD
   // start 40 us late: the first ones hold every primary by then (10 us), and
   // two half-empty waves on a SIMD take longer than one (2000 He histories:
-  // 4.4 -> 3.4 ms).  In a larger one the blocks start over 0.27 ms: started
-  // together, the waves empty their lanes and crowd the shared words together
-  // (2e5 He histories 30 -> 25 ms, 1e6 with wave roles 100 -> 88 ms).  One
-  // nap is 1.07 us.
+  // 4.4 -> 3.4 ms).  In a larger one the blocks start one after another
+  // (plan_admission says over how many naps).  One nap is 1.07 us.
   {
-    const int naps = P.admit_share == 0 ? (int)((blockIdx.x << 8) / gridDim.x)
+    const int naps = P.admit_share == 0 ? (int)((blockIdx.x * (unsigned)P.stagger) / gridDim.x)
                      : P.late_block > 0 && (int)blockIdx.x >= P.late_block ? 38 : 0;
     for (int z = 0; z < naps; ++z) __builtin_amdgcn_s_sleep(40);
   }

@@ -89,9 +89,10 @@ struct AdmitPlan {
   bool strict = false;       // cascades reserved before they start
   int share = 0;             // small batch: primaries a wave admits at once, without the budget
   int late_block = 0;        // small batch: first block to start late (0: none)
+  int stagger = 0;           // naps over which the blocks of another batch start
   double budget = 0.0;       // flights of live cascades
   long long live_floor = 0;  // cascades that may always be live
-  double live_cap = 0.0;     // cascades that may be live at most
+  double live_cap = 1e18;    // cascades that may be live at most
 };
 
 constexpr uint64_t kMaxQueue = uint64_t(1) << 27;  // most queue slots a run takes by itself
@@ -126,18 +127,25 @@ inline AdmitPlan plan_admission(const BatchWork& b, uint64_t qcap, int waves, in
     p.share = int((b.n + first - 1) / first);
     p.late_block = waves > first ? first * 64 / block : 0;
   }
+  const double d = std::min(b.direct_max, 2.0 * b.direct_all / std::max(n, 1.0));
+  const double cap = roomy ? 1e18 : (0.9 * slots + 0.5 * stack_cap * waves) / std::max(d, 1.0);
+  // The blocks of a large batch start over 256 naps (0.27 ms): started together,
+  // the waves empty their lanes and crowd the shared words together (2e5 He
+  // histories 30 -> 24 ms, 2e5 of 1 keV Cu 5.9 -> 5.6).  With fewer primaries than
+  // lanes the first blocks would take them all, 64 a wave: over 48 naps 1e5 He
+  // histories take 11.6 ms, over 256 21 to 26, started together 12 to 13; 7e4 of
+  // 1 keV Cu 1.9, 2.2, 2.0 ms (256 x 3 blocks: 2.6, 3.1, 2.6).
+  p.stagger = n >= lanes ? 256 : 48;
   // With wave roles, a batch of which the feeders' first admission takes nearly
   // all is not held back for the rest: feeders that wait for the budget poll
   // four words that every wave writes (2e5 He histories: 47 against 29 ms).
   const bool feed_all = feeders64 > 0 && b.n <= 128ll * waves;
   p.budget = (feed_all ? 4.0 : 0.5) * slots;
   p.live_floor = waves;
-  p.live_cap = 1e18;
   if (p.strict) {
     p.budget = std::min(12.0 * slots + 1024.0 * waves, 7.5 * slots + 6144.0 * waves);
     p.live_floor = std::min(512, waves);
-    const double d = std::min(b.direct_max, 2.0 * b.direct_all / std::max(n, 1.0));
-    p.live_cap = (0.9 * slots + 0.5 * stack_cap * waves) / std::max(d, 1.0);
+    p.live_cap = cap;
   }
   return p;
 }

@@ -62,7 +62,7 @@ def test_direct_estimate(check, ion, E, target, n):
 def plan(check, n, flights, d, qcap, waves=2048, block=256, stack=128, feeders=0, d_all=None):
     v = check("plan %d %r %r %r %d %d 1024 %d %d %d" % (n, flights, n * d if d_all is None else d_all, d, qcap, waves,
                                                         block, stack, feeders))
-    return dict(zip(("strict", "share", "late", "budget", "floor", "cap"), v))
+    return dict(zip(("strict", "share", "late", "budget", "floor", "cap", "stagger"), v))
 
 
 # measured per live cascade: flights, direct recoils, the part of the direct ones
@@ -102,6 +102,19 @@ def test_rules_at_their_edges(check):
     assert p["strict"] and p["floor"] == 512 and p["cap"] < 512
     assert plan(check, 1000, 1e6, 1e5, 1 << 16, waves=256)["floor"] == 256
     assert plan(check, 1000, 10.0, 3.0, 1 << 16, feeders=20)["share"] == 0
+
+
+# the blocks start one after another only where there is a primary for each lane
+@pytest.mark.parametrize("waves", [2048, 3072])
+@pytest.mark.parametrize("feeders", [0, 62])
+def test_few_primaries_are_not_left_to_the_first_blocks(check, waves, feeders):
+    for n in (65537, 64 * waves - 1):
+        p = plan(check, n, 104.0, 30.0, 1 << 27, waves=waves, feeders=feeders)
+        # 64 primaries per wave: the waves that start before the last is taken
+        # are not a small part of the launch (a nap is 1.07 us, an admission some 10)
+        assert p["stagger"] <= 48 and not p["share"] and not p["strict"]
+    if feeders == 0:
+        assert plan(check, 64 * waves, 104.0, 30.0, 1 << 27, waves=waves)["stagger"] == 256
 
 
 # light ions whose direct recoils overflowed 2^21 slots, or nearly did
