@@ -978,6 +978,7 @@ static void fill_params(Params& P, const mt_ctx* ctx, const mt_primaries* pk, co
   P.f_init = work.flights;
   P.c_floor = plan.live_floor;
   P.c_cap = (long long)std::max(plan.live_cap, double(plan.live_floor));
+  P.first_live = (long long)std::max(plan.first_live, double(plan.live_floor));
   P.stagger = plan.stagger;
   P.h_out = M.h_out;
   P.max_ic = 10000000;

@@ -136,11 +136,11 @@ struct Params {
   // cascade budget: admitted-but-incomplete cascades times the flights per
   // cascade (f_init until 64 cascades completed, then flights ended per
   // completed cascade, an overestimate) stays below `budget`; c_floor cascades
-  // may always be live, c_cap at most.  A queue that has room for what starts at
+  // may always be live, c_cap at most, first_live until 64 have completed.  A queue that has room for what starts at
   // once is budgeted half its entries, unreserved; else each cascade is reserved
   // before it starts (admit_strict; plan_admission in mt_tune.h)
   double budget, f_init;
-  long long c_floor, c_cap;
+  long long c_floor, c_cap, first_live;
   int* h_out;                   // per history: flights queued or running
   int primary_waves64;          // waves per 64 that feed primaries (0: all waves do everything)
   long long max_ic;             // collisions per flight before kErrRunaway

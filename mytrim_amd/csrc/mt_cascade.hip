@@ -428,7 +428,8 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           const uint64_t done = ld_relaxed(&ctrl[kCascDone]);
           const double fhat =
               done >= 64ull ? (double)ld_relaxed(&ctrl[kFlightsEnded]) / (double)done : A->f_init;
-          const long long cmax = min(max((long long)(A->budget / fmax(fhat, 1.0)), A->c_floor), A->c_cap);
+          const long long most_live = done >= 64ull ? A->c_cap : min(A->c_cap, A->first_live);
+          const long long cmax = min(max((long long)(A->budget / fmax(fhat, 1.0)), A->c_floor), most_live);
           const long long n = min((long long)most, cmax - (long long)live);
           if (!A->admit_strict) {
             if (!first_adm || roles) return n;

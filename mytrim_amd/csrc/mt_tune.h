@@ -93,6 +93,7 @@ struct AdmitPlan {
   double budget = 0.0;       // flights of live cascades
   long long live_floor = 0;  // cascades that may always be live
   double live_cap = 1e18;    // cascades that may be live at most
+  double first_live = 1e18;  // and at most until 64 cascades have ended
 };
 
 constexpr uint64_t kMaxQueue = uint64_t(1) << 27;  // most queue slots a run takes by itself
@@ -136,12 +137,29 @@ inline AdmitPlan plan_admission(const BatchWork& b, uint64_t qcap, int waves, in
   // histories take 11.6 ms, over 256 21 to 26, started together 12 to 13; 7e4 of
   // 1 keV Cu 1.9, 2.2, 2.0 ms (256 x 3 blocks: 2.6, 3.1, 2.6).
   p.stagger = n >= lanes ? 256 : 48;
-  // With wave roles, a batch of which the feeders' first admission takes nearly
-  // all is not held back for the rest: feeders that wait for the budget poll
-  // four words that every wave writes (2e5 He histories: 47 against 29 ms).
-  const bool feed_all = feeders64 > 0 && b.n <= 128ll * waves;
-  p.budget = (feed_all ? 4.0 : 0.5) * slots;
+  p.budget = 0.5 * slots;
   p.live_floor = waves;
+  if (feeders64 > 0 && !p.strict) {
+    // With wave roles the feeders' first admission is what counts.  A batch that it
+    // takes nearly whole (64 a feeder) is not held back for the rest: feeders that
+    // wait for the budget poll four words that every wave writes (2e5 He histories,
+    // 62 feeders of 64: 47 against 32 ms).  A larger one floods the queue before the
+    // few other waves have taken anything in, so until 64 cascades have ended 16 per
+    // wave may be live (4e5 He histories 62 -> 46 ms, 3e5 of 2 MeV C in W 167 -> 150);
+    // after that 224 per wave, counted by the flights expected, as far as the queue
+    // bears it (1e6: 114 -> 84 ms unbounded against so, and 522 -> 460).  Blocks over
+    // 256 naps: 1e5 He 27 ms, over 8 17; the larger ones over 16.
+    const double feeders = waves * (feeders64 / 64.0);
+    if (n <= 96.0 * feeders) {
+      p.budget = 4.0 * slots;
+      p.stagger = 8;
+    } else {
+      p.budget = std::min(std::max(0.5 * slots, 224.0 * waves * b.flights), 7.5 * slots + 6144.0 * waves);
+      p.live_cap = cap;
+      p.first_live = 16.0 * waves;
+      p.stagger = 16;
+    }
+  }
   if (p.strict) {
     p.budget = std::min(12.0 * slots + 1024.0 * waves, 7.5 * slots + 6144.0 * waves);
     p.live_floor = std::min(512, waves);

@@ -1,7 +1,7 @@
 // Reads lines of stdin.  "direct Z1 m1 E Z2 m2 Ed" prints direct_estimate;
 // "plan n flights direct_all direct_max qcap waves simds block stack feeders"
 // prints plan_admission's strict share late_block budget live_floor live_cap
-// stagger.
+// stagger first_live.
 #include <cstdio>
 #include <cstring>
 
@@ -23,8 +23,8 @@ int main() {
                      &simds, &block, &stack, &k) != 10)
         return 1;
       const mt::AdmitPlan p = mt::plan_admission(b, qcap, w, simds, block, stack, k);
-      std::printf("%d %d %d %.17g %lld %.17g %d\n", int(p.strict), p.share, p.late_block, p.budget, p.live_floor,
-                  p.live_cap, p.stagger);
+      std::printf("%d %d %d %.17g %lld %.17g %d %.17g\n", int(p.strict), p.share, p.late_block, p.budget, p.live_floor,
+                  p.live_cap, p.stagger, p.first_live);
     }
   }
 }

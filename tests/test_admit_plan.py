@@ -62,7 +62,7 @@ def test_direct_estimate(check, ion, E, target, n):
 def plan(check, n, flights, d, qcap, waves=2048, block=256, stack=128, feeders=0, d_all=None):
     v = check("plan %d %r %r %r %d %d 1024 %d %d %d" % (n, flights, n * d if d_all is None else d_all, d, qcap, waves,
                                                         block, stack, feeders))
-    return dict(zip(("strict", "share", "late", "budget", "floor", "cap", "stagger"), v))
+    return dict(zip(("strict", "share", "late", "budget", "floor", "cap", "stagger", "first"), v))
 
 
 # measured per live cascade: flights, direct recoils, the part of the direct ones
@@ -115,6 +115,43 @@ def test_few_primaries_are_not_left_to_the_first_blocks(check, waves, feeders):
         assert p["stagger"] <= 48 and not p["share"] and not p["strict"]
     if feeders == 0:
         assert plan(check, 64 * waves, 104.0, 30.0, 1 << 27, waves=waves)["stagger"] == 256
+
+
+# with wave roles: the feeders' first admission takes the batch (64 a feeder, half as
+# many again) and nothing is held back, or the first cascades are few
+def test_feeders_take_a_batch_or_start_slowly(check):
+    he = lambda n, **kw: plan(check, n, 104.0, 30.0, 1 << 27, waves=3072, feeders=62, **kw)
+    feeder_waves = 3072 * 62 // 64
+    for n in (100, 2 * 10 ** 5, 96 * feeder_waves):
+        assert he(n)["first"] > n and he(n)["budget"] >= 104.0 * n and he(n)["stagger"] <= 16
+    for n in (96 * feeder_waves + 1, 4 * 10 ** 5, 10 ** 6):
+        p = he(n)
+        assert p["first"] == 16 * 3072 and p["stagger"] <= 16 and not p["strict"]
+        # never more flights, nor direct recoils, than the queue bears
+        assert p["budget"] <= 7.5 * (1 << 27) + 6144 * 3072
+        assert p["budget"] / 104.0 * 30.0 < 1 << 27
+    # long cascades: the queue's share, not 224 cascades per wave
+    p = plan(check, 10 ** 6, 48618.0, 373.0, 1 << 27, waves=3072, feeders=10, d_all=4e7)
+    assert p["budget"] == 7.5 * (1 << 27) + 6144 * 3072 and p["cap"] * 80.0 < 1.01 * (1 << 27)
+    # without roles, and where the cascades are reserved, nothing of this
+    assert plan(check, 10 ** 6, 104.0, 30.0, 1 << 27, waves=3072)["first"] > 1e17
+    assert plan(check, 10 ** 6, 104.0, 30.0, 1 << 21, waves=3072, feeders=62)["first"] > 1e17
+
+
+# batches on both sides of what the feeders take at once: the same results
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_hist", [61440, 61441, 150000])
+def test_batches_around_the_feeders_first_admission(n_hist):
+    from mytrim_amd import gpu
+    prob = configs.vacancy_case("cu", 1e3, n_hist, seed=13)
+    e = gpu.Engine(0)
+    try:
+        ref = e.run(prob)
+        for k in (1, 20, 62):
+            e.tune(primary_waves64=k)
+            assert_same(ref, e.run(prob))
+    finally:
+        e.close()
 
 
 # light ions whose direct recoils overflowed 2^21 slots, or nearly did
