@@ -133,10 +133,12 @@ inline AdmitPlan plan_admission(const BatchWork& b, uint64_t qcap, int waves, in
   // The blocks of a large batch start over 256 naps (0.27 ms): started together,
   // the waves empty their lanes and crowd the shared words together (2e5 He
   // histories 30 -> 24 ms, 2e5 of 1 keV Cu 5.9 -> 5.6).  With fewer primaries than
-  // lanes the first blocks would take them all, 64 a wave: over 48 naps 1e5 He
-  // histories take 11.6 ms, over 256 21 to 26, started together 12 to 13; 7e4 of
-  // 1 keV Cu 1.9, 2.2, 2.0 ms (256 x 3 blocks: 2.6, 3.1, 2.6).
-  p.stagger = n >= lanes ? 256 : 48;
+  // lanes the first blocks would take them all, 64 a wave: 1e5 He histories take 12 ms
+  // over 48 or 8 naps, 21 to 26 over 256; 7e4 of 1 keV Cu 2.0, 2.0 and 2.2 ms, 1e5 3.1,
+  // 2.3 and 3.1, 7e4 He 9.0, 9.9 and 9.0, 7e4 of 2 MeV C in W 37, 42 and 59.  With three
+  // waves per SIMD 8 naps are better: 1e5 He 20, 19 and 27 ms, 1.4e5 21, 20 and 39,
+  // 1.4e5 of 1 keV Cu 4.2, 3.2 and 4.3.
+  p.stagger = n >= lanes ? 256 : waves > 2 * simds ? 8 : 48;
   p.budget = 0.5 * slots;
   p.live_floor = waves;
   if (feeders64 > 0 && !p.strict) {
