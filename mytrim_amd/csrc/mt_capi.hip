@@ -892,17 +892,20 @@ static BatchWork batch_work(const mt_ctx* ctx, const PrimaryStats& st, const mt_
                             uint64_t qcap) {
   BatchWork b;
   b.n = n;
-  b.flights = flights;
+  b.flights = b.flights_mean = flights;
   if (double(n) * flights <= 2.0 * double(qcap) || o->follow_max_gen == 0 || o->follow_max_gen == 1) return b;
   double ed_min = 1e300;
   for (const HostMaterial& m : ctx->tgt.mat)
     for (const HostElement& e : m.el) ed_min = std::min(ed_min, e.Edisp);
+  b.flights_mean = 0.0;
   for (int s = 0; s < st.n; ++s) {
-    double mean = 0.0, most = 0.0;
+    double mean = 0.0, most = 0.0, f = 1.0;
     for (const HostMaterial& m : ctx->tgt.mat) {
+      f = std::max(f, flights_estimate(st.Z[s], st.m[s], st.e_sum[s] / st.num[s], m.az, m.am, ed_min));
       mean = std::max(mean, direct_estimate(st.Z[s], st.m[s], st.e_sum[s] / st.num[s], m.az, m.am, ed_min));
       most = std::max(most, direct_estimate(st.Z[s], st.m[s], st.e_max[s], m.az, m.am, ed_min));
     }
+    b.flights_mean += f * st.num[s] / double(n);
     b.direct_all += st.num[s] * mean;
     b.direct_max = std::max(b.direct_max, most);
   }
@@ -975,7 +978,7 @@ static void fill_params(Params& P, const mt_ctx* ctx, const mt_primaries* pk, co
   P.admit_share = plan.share;
   P.late_block = plan.late_block;
   P.budget = plan.budget;
-  P.f_init = work.flights;
+  P.f_init = plan.flights;
   P.c_floor = plan.live_floor;
   P.c_cap = (long long)std::max(plan.live_cap, double(plan.live_floor));
   P.first_live = (long long)std::max(plan.first_live, double(plan.live_floor));

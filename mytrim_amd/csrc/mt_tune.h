@@ -77,11 +77,11 @@ inline double direct_estimate(double Z1, double m1, double E, double Z2, double 
   return sum;
 }
 
-// What a batch is expected to bring: flights per cascade, direct recoils of all
-// its primaries and of the one with the most.
+// What a batch is expected to bring: flights of the largest cascade and of the mean
+// one, direct recoils of all its primaries and of the one with the most.
 struct BatchWork {
   long long n = 0;
-  double flights = 1.0, direct_all = 0.0, direct_max = 0.0;
+  double flights = 1.0, flights_mean = 1.0, direct_all = 0.0, direct_max = 0.0;
 };
 
 // How a launch admits its primaries (see Params)
@@ -91,6 +91,7 @@ struct AdmitPlan {
   int late_block = 0;        // small batch: first block to start late (0: none)
   int stagger = 0;           // naps over which the blocks of another batch start
   double budget = 0.0;       // flights of live cascades
+  double flights = 1.0;      // a cascade's, until 64 have ended
   long long live_floor = 0;  // cascades that may always be live
   double live_cap = 1e18;    // cascades that may be live at most
   double first_live = 1e18;  // and at most until 64 cascades have ended
@@ -140,6 +141,7 @@ inline AdmitPlan plan_admission(const BatchWork& b, uint64_t qcap, int waves, in
   // 1.4e5 of 1 keV Cu 4.2, 3.2 and 4.3.
   p.stagger = n >= lanes ? 256 : waves > 2 * simds ? 8 : 48;
   p.budget = 0.5 * slots;
+  p.flights = b.flights;
   p.live_floor = waves;
   if (feeders64 > 0 && !p.strict) {
     // With wave roles the feeders' first admission is what counts.  A batch that it
@@ -164,8 +166,15 @@ inline AdmitPlan plan_admission(const BatchWork& b, uint64_t qcap, int waves, in
   }
   if (p.strict) {
     p.budget = std::min(12.0 * slots + 1024.0 * waves, 7.5 * slots + 6144.0 * waves);
-    p.live_floor = std::min(512, waves);
     p.live_cap = cap;
+    // The first cascades of a mixed batch are hardly all of its largest kind.  What may
+    // start at first may stay live: the measured flights per cascade count those of
+    // unfinished ones too (20 000 histories of H to Xe ions, 10 keV to 2 MeV, through
+    // 2^21 slots: 54 ms with 561 live at first and 512 later, 50 with 1900; all at once
+    // they take 37, but with twice as many live 1e5 of them, heaviest first, overflow)
+    p.flights = std::min(b.flights, 4.0 * b.flights_mean);
+    p.live_floor = (long long)std::max(std::min(512.0, double(waves)),
+                                       std::min(std::min(double(waves), p.budget / p.flights), cap));
   }
   return p;
 }

@@ -22,6 +22,7 @@ int main() {
       if (std::scanf("%lld %lf %lf %lf %llu %d %d %d %d %d", &b.n, &b.flights, &b.direct_all, &b.direct_max, &qcap, &w,
                      &simds, &block, &stack, &k) != 10)
         return 1;
+      b.flights_mean = b.flights;
       const mt::AdmitPlan p = mt::plan_admission(b, qcap, w, simds, block, stack, k);
       std::printf("%d %d %d %.17g %lld %.17g %d %.17g\n", int(p.strict), p.share, p.late_block, p.budget, p.live_floor,
                   p.live_cap, p.stagger, p.first_live);

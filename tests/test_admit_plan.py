@@ -6,6 +6,7 @@ import os
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 import oracle_lib as O
@@ -98,6 +99,9 @@ def test_rules_at_their_edges(check):
         assert p["share"] == (0 if n > 65536 else -(-n // 1024)) and not p["strict"]
     assert plan(check, 4096, 1024.0, 30.0, STATIC_SLOTS)["strict"] == 0  # twice the slots
     assert plan(check, 4097, 1024.0, 30.0, STATIC_SLOTS)["strict"] == 1
+    # what may start at first may stay live: 512 at least, a wave each at most
+    assert plan(check, 10 ** 6, 8010.0, 184.0, STATIC_SLOTS)["floor"] == 2048
+    assert plan(check, 10 ** 6, 48618.0, 373.0, STATIC_SLOTS)["floor"] == int((12 * STATIC_SLOTS + 1024 * 2048) / 48618.0)
     p = plan(check, 1000, 1e6, 1e5, 1 << 16)
     assert p["strict"] and p["floor"] == 512 and p["cap"] < 512
     assert plan(check, 1000, 1e6, 1e5, 1 << 16, waves=256)["floor"] == 256
@@ -165,6 +169,23 @@ def test_light_ions_through_the_static_queue(ion, E, target, n):
         ref, r = e.run(prob), e.run(prob, noalloc=True)
         assert_same(ref, r)
         assert r["queue_peak"] < 0.9 * STATIC_SLOTS / 16
+    finally:
+        e.close()
+
+
+# mixed ions, as drawn and with the largest cascades first
+@pytest.mark.gpu
+@pytest.mark.parametrize("heaviest_first", [False, True])
+def test_mixed_ions_through_the_static_queue(heaviest_first):
+    from mytrim_amd import gpu
+    prob = configs.c4_mixed_uo2(100000, seed=3, w=4000.0, geometry_seed=2345)
+    if heaviest_first:
+        q = prob.primaries
+        o = np.lexsort((-q.E, -q.Z))
+        prob = prob.with_(primaries=dataclasses.replace(q, Z=q.Z[o], m=q.m[o], E=q.E[o], pos=q.pos[o], dir=q.dir[o]))
+    e = gpu.Engine(0)
+    try:
+        assert_same(e.run(prob), e.run(prob, noalloc=True))
     finally:
         e.close()
 
