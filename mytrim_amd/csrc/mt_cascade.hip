@@ -803,8 +803,8 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
         }
         // fate of recoil and ion (trim.C:357-411)
         // to nuclear losses from the recoil, added where the branches meet; the
-        // ion's rest is a term of its own (the sum of the two would be rounded
-        // before the compensated addition)
+        // rest of an ion that stops is a term of its own, added where flights end
+        // (the sum of the two would be rounded before the compensated addition)
         double enuc = 0.0;
         if (lost) {
           state = 4;
@@ -850,14 +850,10 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
           } else {
             // replacementCollision (trim.C:388-395)
             state = (H->species[F.sp].Z == ec.Z) ? 1 : 2;
-            kadd(enuc_s, enuc_e, F.E);
           }
         } else {
           enuc = rE + ec.Elbind;
-          if (F.E < C->Ef) {
-            state = 3;
-            kadd(enuc_s, enuc_e, F.E);
-          }
+          if (F.E < C->Ef) state = 3;
         }
         kadd(enuc_s, enuc_e, enuc);
         ended = state > 0;
@@ -1105,6 +1101,7 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
       if (lane == 0 && fe_pending >= 256ull) atomicAdd(&ctrl[kFlightsEnded], fe_pending);
       if (fin) {
         ++l_flight32;
+        if (state > 0 && state < 4) kadd(enuc_s, enuc_e, F.E);
         l_coll32 += (unsigned)(vacuum ? F.ic - 1 : F.ic);
         l_coll0_32 += F.gen == 0 ? (unsigned)(vacuum ? F.ic - 1 : F.ic) : 0u;
         l_vacuum32 += vacuum ? 1u : 0u;
