@@ -252,8 +252,8 @@ __device__ __forceinline__ void physics(const TableView& T, int sp, int k, doubl
 
 }  // namespace
 
-// Three waves per SIMD (168 VGPRs): the FP64 and FP32 kernels fit without
-// spills (the per-history FP64 variants spill a few dwords); the surrogate
+// Three waves per SIMD (168 VGPRs): the FP32 kernels fit without spills, the
+// FP64 ones spill one register (the per-history variants a few); the surrogate
 // kernels, whose network needs more registers, keep two.
 template <int ARITH, int POT, int GEO, bool PERHIST>
 __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascade_kernel(Params P) {
@@ -307,7 +307,8 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
   unsigned long long* ctrl = P.ctrl;
   const unsigned long long clk0 = (unsigned long long)clock64();
   const unsigned long long wall0 = (unsigned long long)wall_clock64();
-  // wave 0 stamps the launch (all waves start within a microsecond)
+  // wave 0 stamps the launch: the first blocks start together, those that do not
+  // fit the device at once when others have left
   if (blockIdx.x == 0 && threadIdx.x == 0)
     __hip_atomic_store(&ctrl[kT0], wall0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 

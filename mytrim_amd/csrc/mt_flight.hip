@@ -56,7 +56,7 @@ struct FlightPending {
 // by wave 3 only; it draws again as the reference does and the slot is repeated
 // with the draws that follow.
 // A collision took 15 000 cycles on one lane with each uniform loaded where it
-// was drawn, and takes 7500 (a 500 keV Cu flight of 580: 3.7 -> 1.9 ms): wave 0's
+// was drawn, and takes 7500 (the call of a 500 keV Cu flight: 3.4 -> 1.8 ms): wave 0's
 // 5500, of which the library's power and the divisions are a third, and 1900 of
 // merging, mostly LDS latency.  Waves 1, 2 and 3 need 2400, 1500 and 3900.
 template <int POT>
