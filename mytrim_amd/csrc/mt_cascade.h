@@ -74,7 +74,8 @@ enum ErrBits {
   kErrBadEntry = 4,   // queue entry failed validation
   kErrTimeout = 8,    // a wait exceeded the wall-clock limit
   kErrNewton = 16,    // Newton solve hit its iteration cap
-  kErrNonFinite = 32  // a flight's energy or position became NaN or infinite
+  kErrNonFinite = 32, // a flight's energy or position became NaN or infinite
+  kErrLeft = 64       // (beside another) a wave left a claimed entry of an aborted run
 };
 
 enum Counter {

@@ -550,12 +550,16 @@ __global__ void __launch_bounds__(kCascadeMaxBlock, (ARITH == 2 ? 2 : 3)) cascad
                   break;
                 }
                 if (ld_relaxed(&ctrl[kError]) != 0ull) {  // another wave aborted the run
+                  // The entry may never be published, and the lane's stack slot
+                  // holds an older flight: run again, its recoils would go to the
+                  // full queue again, without end.  This wave takes in no more.
+                  err |= kErrLeft;
                   mine = false;
                   break;
                 }
               }
             }
-            const uint64_t bad = __ballot((err & (kErrTimeout | kErrBadEntry)) != 0u);
+            const uint64_t bad = __ballot((err & (kErrTimeout | kErrBadEntry | kErrLeft)) != 0u);
             if (bad == 0ull) {
               scount += (int)got;
             } else if (lane == __ffsll((long long)bad) - 1) {  // abort the run: every wave leaves
